@@ -118,7 +118,7 @@ def build_oracle() -> None:
 def build_reference_host() -> None:
     """Compiles the reference's host-only headers (oracle/_ref), if present."""
     recipe = ROOT / "oracle" / "ref_host.mk"
-    if Path("/root/reference").is_dir() and recipe.exists():
+    if Path("/root/reference/include").is_dir() and recipe.exists():
         _run(["make", "-B", "-f", str(recipe), "-C", str(ROOT / "oracle")])
 
 
