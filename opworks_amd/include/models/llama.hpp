@@ -728,7 +728,8 @@ template <typename WT> class LlamaModelT final : public LlamaRuntime {
     // bf16 on load from 16 rows (the reference's linear_mma_bf16 path,
     // models/llama.cuh:190-199), and below 16 rows the fp32 MFMA GEMM with fp32
     // inputs against the widened bf16 weights, as the reference's linear_dispatch does.
-    // Outputs with too few tiles to fill the GPU (o_proj, down, qkv at a few
+    // Up to 64 rows every form runs on gemm_rows_kernel, which splits K inside its workgroups.
+    // Above, outputs with too few tiles to fill the GPU (o_proj, down, qkv at a few
     // hundred rows) split K across workgroups into the session's workspace.
     // `reduce` (optional, split-K outputs): run in place of the split-K reduction kernel, see
     // gemm_f32_launch_splitk. Returns true when K was split (and `reduce`, if given, ran).

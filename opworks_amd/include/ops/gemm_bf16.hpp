@@ -526,12 +526,18 @@ __global__ __launch_bounds__(Shape::kThreads) void gemm_bf16_mfma_kernel(const T
 }
 
 // C written per kStore (see GemmStore): store, += (residual), or SwiGLU of
-// interleaved (gate, up) column pairs into C[M][N / 2].
+// interleaved (gate, up) column pairs into C[M][N / 2]. Up to 64 rows take gemm_rows_kernel.
 template <typename TA, typename Epi, GemmStore kStore = GemmStore::store>
 void gemm_bf16_launch(const TA *A, const uint16_t *W, const float *bias, float *C, int M, int N, int K, Epi epi,
                       hipStream_t stream, int splits = 1) {
     require((kStore != GemmStore::swiglu && kStore != GemmStore::swiglu_bf16) || N % 2 == 0,
             "swiglu epilogue needs an even number of columns");
+    if constexpr (kStore != GemmStore::partial) {
+        if (splits == 1 && gemm_rows_use(M, K)) {
+            gemm_rows_launch<std::is_same_v<TA, float>, Epi, kStore>(A, W, bias, C, M, N, K, epi, stream);
+            return;
+        }
+    }
     const int tiles = static_cast<int>(blocks_for64(M, kBfBM) * blocks_for64(N, kBfBN));
     const dim3 grid(tiles, splits);
     const bool vec = aligned16(A) && aligned16(W) && K % 8 == 0;
@@ -555,8 +561,8 @@ void gemm_bf16_launch_splitk(const TA *A, const uint16_t *W, const float *bias, 
                              Epi epi, float *ws, int64_t ws_floats, hipStream_t stream) {
     const int tiles = static_cast<int>(blocks_for64(M, kBfBM) * blocks_for64(N, kBfBN));
     const int splits = splitk_factor(tiles, static_cast<int>(blocks_for64(K, kBfBK)), 256);
-    if (splits == 1 || N % 4 != 0 || !ws || int64_t(splits) * M * N > ws_floats || !aligned16(C) ||
-        (bias && !aligned16(bias))) {
+    if (splits == 1 || gemm_rows_use(M, K) || N % 4 != 0 || !ws || int64_t(splits) * M * N > ws_floats ||
+        !aligned16(C) || (bias && !aligned16(bias))) {
         gemm_bf16_launch<TA, Epi, kStore>(A, W, bias, C, M, N, K, epi, stream);
         return;
     }
@@ -568,7 +574,7 @@ void gemm_bf16_launch_splitk(const TA *A, const uint16_t *W, const float *bias, 
 
 // bf16 A on the direct path (both operands straight into LDS), for any M: 256 x 256 tiles when
 // they fill the GPU's 256 CUs, else 128 x 256 three-stage tiles from 256 rows (one workgroup per
-// CU) and 128 x 128 tiles below (two per CU), and for store / residual outputs K split across
+// CU), 128 x 128 tiles below (two per CU) and gemm_rows_kernel up to 64 rows, and for store / residual outputs K split across
 // workgroups toward one round of the GPU, at least 8 K tiles of 64 per split, the partial tiles
 // summed in split order by splitk_reduce_kernel. At M = 512 (a 512-token prefill) the 256 x 256
 // tiles gave gate/up 128 workgroups and qkv, o_proj and down 8-way splits on 16-24 tiles.
@@ -581,6 +587,10 @@ bool gemm_bf16_launch_direct(const uint16_t *A, const uint16_t *W, const float *
     const int big_tiles = static_cast<int>(blocks_for64(M, kBfBM) * blocks_for64(N, kBfBN));
     constexpr bool kSwiglu = kStore == GemmStore::swiglu || kStore == GemmStore::swiglu_bf16;
     require(!kSwiglu || N % 2 == 0, "swiglu epilogue needs an even number of columns");
+    if (gemm_rows_use(M, K)) { // few rows: K is split inside the workgroups
+        gemm_bf16_launch<uint16_t, Epi, kStore>(A, W, bias, C, M, N, K, epi, stream);
+        return false;
+    }
     if (!vec || big_tiles >= 256) {
         if constexpr (kSwiglu)
             gemm_bf16_launch<uint16_t, Epi, kStore>(A, W, bias, C, M, N, K, epi, stream);

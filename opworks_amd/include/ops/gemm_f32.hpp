@@ -487,6 +487,7 @@ void gemm_f32_launch_shape(const float *A, const TB *B, const float *bias, float
 
 } // namespace opworks::detail
 
+#include "gemm_rows.hpp"
 #include "gemm_x6.hpp"
 
 namespace opworks::detail {
@@ -518,6 +519,7 @@ inline bool gemm_use_x6(const float *A, const TB *B, int M, int N, int K) {
 }
 
 // Enqueues C[M][N] = epi(A[M][K] B + bias) (written per kStore). K == 0 writes epi(bias or 0).
+// Up to 64 rows of an nk-layout product take gemm_rows_kernel.
 // When K is not split: GemmBig when its tiles alone cover every CU, else GemmMid when its
 // 256 x 128 tiles do (the prefill gate/up projection at 512 rows: 280 -> 262 us against
 // GemmSmall); otherwise, and for split-K partials, GemmSmall.
@@ -526,6 +528,12 @@ template <BLayout kB, typename Epi, GemmStore kStore = GemmStore::store, typenam
 void gemm_f32_launch(const float *A, const TB *B, const float *bias, float *C, int M, int N, int K, Epi epi,
                      hipStream_t stream, int splits = 1, bool allow_x6 = true) {
     require(kStore != GemmStore::swiglu || N % 2 == 0, "swiglu epilogue needs an even number of columns");
+    if constexpr (kB == BLayout::nk && kAL == ALayout::mk && kStore != GemmStore::partial) {
+        if (splits == 1 && gemm_rows_use(M, K)) {
+            gemm_rows_launch<false, Epi, kStore>(A, B, bias, C, M, N, K, epi, stream);
+            return;
+        }
+    }
     if constexpr (std::is_same_v<TB, float> && kAL == ALayout::mk &&
                   (kStore == GemmStore::store || kStore == GemmStore::swiglu)) {
         if (allow_x6 && gemm_use_x6<kB, kStore, TB, kAL>(A, B, M, N, K)) {
@@ -558,6 +566,10 @@ bool gemm_f32_launch_splitk(const float *A, const TB *B, const float *bias, floa
     // K at all, else on GemmSmall tiles up to 512 (prefill at 512 rows: qkv 86.2 -> 81.8 us, down
     // 152.5 -> 148.4 us, o_proj unchanged). Either plan needs at most 256 * 256 * 128 =
     // 512 * 128 * 128 floats.
+    if (kB == BLayout::nk && gemm_rows_use(M, K)) { // splits K inside its workgroups
+        gemm_f32_launch<kB, Epi, kStore, TB>(A, B, bias, C, M, N, K, epi, stream, 1, false);
+        return false;
+    }
     const int ktiles = static_cast<int>(blocks_for64(K, kGemmBK));
     const int mid_splits =
         M >= GemmMid::BM

@@ -1,0 +1,402 @@
+#pragma once
+
+// GEMM for few rows: C[m][n] = epi(sum_k X[m][k] W[n][k] + bias[n]) with W in the HF [n][k] layout.
+//
+// The tiled kernels stage 128 x 128 or larger tiles through LDS for all of a workgroup's waves, so a
+// product of a few rows (a decode batch, a short prompt) multiplies mostly padding on N / 128
+// workgroups. Here the weight stream is the bound. A workgroup owns 16 FM rows x 16 FN columns of C,
+// its kWaves waves take the K steps round robin, and their accumulators are summed through LDS in wave
+// order at the end (the result does not depend on timing): N / 16 workgroups of 4 or 8 waves instead
+// of N / 128.
+//
+// fp32 inputs multiply on v_mfma_f32_16x16x4f32 (bf16 weights widened exactly), bf16 inputs, and fp32
+// inputs rounded to bf16 (kRound), on v_mfma_f32_16x16x32_bf16. Up to 64 rows the fp32 MFMAs take
+// less time than the weights' bytes; three bf16 parts per operand took longer (8 x 2048 against
+// 8192 x 2048: 16.1 against 14.4 us), since every workgroup splits X again.
+//
+// A wave stages its own K steps of 128 bytes per row in a ring of kDepth stages with direct loads
+// (global_load_lds_dwordx4, 8 rows x 128 contiguous bytes per instruction) and reads its fragments
+// from there; no barrier, as no other wave reads them. Loads straight into fragments touch 16 rows
+// per 16 lanes and ran at 16 bytes a cycle per CU (8 x 8192 against 2048 x 8192: 25.7 against 20.5
+// us). They remain for operands that are not 16-byte aligned row by row (kStaged false), on
+// 16-byte loads at the element's own alignment.
+//
+// Measured (fp32 weights, HIP events, weights from HBM; the tiled kernel before): 8 x 2048 against
+// 8192 x 2048 157 -> 14.4 us (67 MB: 4.7 TB/s), 64 rows 157 -> 25; bf16 weights and fp32 inputs
+// rounded to bf16, 32 rows 75 -> 10.9.
+//
+// W is the MFMA's A operand, so a lane ends with 4 consecutive columns of one row.
+
+// Included by gemm_f32.hpp ahead of its launchers; it uses that header's GemmStore.
+
+#include <cstdint>
+#include <type_traits>
+
+#include "../core/bf16x6.hpp" // cvt_pk_bf16, bf16x8v
+#include "../core/hip_utils.hpp"
+#include "../core/lds_direct.hpp"
+
+namespace opworks::detail {
+
+using f32x4u = f32x4 __attribute__((aligned(4))); // 16-byte load at 4-byte alignment
+using u32x4u = u32x4 __attribute__((aligned(2))); // and at 2-byte alignment
+
+// Eight consecutive elements of a row as they are in memory.
+template <typename T> struct Raw8;
+template <> struct Raw8<float> {
+    f32x4 v[2];
+};
+template <> struct Raw8<uint16_t> {
+    u32x4 v;
+};
+__device__ __forceinline__ void raw8_load(Raw8<float> &r, const float *p) {
+    r.v[0] = *reinterpret_cast<const f32x4u *>(p);
+    r.v[1] = *reinterpret_cast<const f32x4u *>(p + 4);
+}
+__device__ __forceinline__ void raw8_load(Raw8<uint16_t> &r, const uint16_t *p) {
+    r.v = *reinterpret_cast<const u32x4u *>(p);
+}
+// The first `count` (<= 8, may be negative) elements at p, zeros after them. p[0] is readable always.
+__device__ __forceinline__ void raw8_load_tail(Raw8<float> &r, const float *p, int count) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const float x = p[j < count ? j : 0];
+        r.v[j / 4][j % 4] = j < count ? x : 0.f;
+    }
+}
+__device__ __forceinline__ void raw8_load_tail(Raw8<uint16_t> &r, const uint16_t *p, int count) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const uint32_t lo = p[2 * j < count ? 2 * j : 0], hi = p[2 * j + 1 < count ? 2 * j + 1 : 0];
+        r.v[j] = (2 * j < count ? lo : 0u) | (2 * j + 1 < count ? hi << 16 : 0u);
+    }
+}
+__device__ __forceinline__ float raw8_at(const Raw8<float> &r, int j) { return r.v[j / 4][j % 4]; }
+__device__ __forceinline__ float raw8_at(const Raw8<uint16_t> &r, int j) {
+    return __uint_as_float(j & 1 ? r.v[j / 2] & 0xffff0000u : r.v[j / 2] << 16);
+}
+// The eight as a bf16 MFMA operand; fp32 rounds to nearest even.
+__device__ __forceinline__ bf16x8v raw8_bf16(const Raw8<float> &r) {
+    return __builtin_bit_cast(bf16x8v, u32x4{cvt_pk_bf16(r.v[0][0], r.v[0][1]), cvt_pk_bf16(r.v[0][2], r.v[0][3]),
+                                             cvt_pk_bf16(r.v[1][0], r.v[1][1]), cvt_pk_bf16(r.v[1][2], r.v[1][3])});
+}
+__device__ __forceinline__ bf16x8v raw8_bf16(const Raw8<uint16_t> &r) { return __builtin_bit_cast(bf16x8v, r.v); }
+
+// Tile shape: 16 FM rows x 16 FN columns per workgroup, kWaves waves over K, kDepth steps in flight.
+template <int kFM, int kFN, int kW, int kD> struct RowsShape {
+    static constexpr int FM = kFM, FN = kFN, kWaves = kW, kDepth = kD, kThreads = kW * kWaveSize;
+};
+
+template <typename S, typename TX, typename TW, bool kRound, bool kStaged, typename Epi, GemmStore kStore>
+__global__ __launch_bounds__(S::kThreads) void gemm_rows_kernel(const TX *__restrict__ X, const TW *__restrict__ W,
+                                                                const float *__restrict__ bias, float *__restrict__ C,
+                                                                int M, int N, int K, Epi epi) {
+    constexpr int FM = S::FM, FN = S::FN, kWaves = S::kWaves, kDepth = S::kDepth;
+    constexpr bool kF32X = std::is_same_v<TX, float>, kF32W = std::is_same_v<TW, float>;
+    static_assert(!kF32W || (kF32X && !kRound), "fp32 weights take fp32 inputs");
+    constexpr bool kF32Mfma = kF32X && !kRound;
+    constexpr int kU = kF32W ? 1 : 2, kStep = 32 * kU; // K step: 128 bytes of each weight row
+    // Staged steps: blocks of 16 rows x 128 bytes, FN of W, then FM x kXB of X.
+    constexpr int kXB = kF32X && !kF32W ? 2 : 1, kXHalf = 128 / int(sizeof(TX)); // X elements per block row
+    constexpr int kBlocks = FN + FM * kXB, kLoads = 2 * kBlocks;                 // blocks, wave loads per step
+    constexpr int kItems = FN * FM * kWaveSize;                                  // f32x4 of the output tile
+    constexpr int kRing = kStaged ? kWaves * kDepth * kBlocks * 2048 : 16, kRed = kWaves * kItems * 16;
+    __shared__ __attribute__((aligned(16))) unsigned char lds[kRing > kRed ? kRing : kRed];
+    const int lane = threadIdx.x % kWaveSize;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
+    const int l16 = lane % 16, quad = lane / 16;
+    const int n0 = blockIdx.x * 16 * FN, m0 = blockIdx.y * 16 * FM;
+    if (kStaged && M < 0) // never: an ordinary store, so the compiler keeps the reads of the direct loads
+        lds[threadIdx.x] = 0;
+
+    // Rows past N or M read the last row: those outputs are not stored.
+    auto w_row = [&](int r) { return W + int64_t(n0 + r < N ? n0 + r : N - 1) * K; };
+    auto x_row = [&](int r) { return X + int64_t(m0 + r < M ? m0 + r : M - 1) * K; };
+
+    struct Frags {
+        Raw8<TW> w[FN][kU];
+        Raw8<TX> x[FM][kU];
+    };
+    // Staged loads: instruction h of a block covers its rows 8 h .. 8 h + 7, lane l row 8 h + l / 8,
+    // 16-byte slot l % 8, which holds chunk (l % 8) ^ ((row >> 1) & 7) of that row's 128 bytes.
+    const int s_row = lane >> 3;
+    const TW *wsrc[FN][2];
+    const TX *xsrc[FM][2];
+    if constexpr (kStaged) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int r = 8 * h + s_row, chunk = (lane & 7) ^ ((r >> 1) & 7);
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+                wsrc[j][h] = w_row(16 * j + r) + chunk * (16 / int(sizeof(TW)));
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+                xsrc[i][h] = x_row(16 * i + r) + chunk * (16 / int(sizeof(TX)));
+        }
+    }
+    auto stage_of = [&](int slot) { return lds + (wave * kDepth + slot) * kBlocks * 2048; };
+    auto stage = [&](int slot, int step) {
+        unsigned char *st = stage_of(slot);
+        const int k = step * kStep;
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                load_lds16(wsrc[j][h] + k, reinterpret_cast<uint16_t *>(st + j * 2048 + h * 1024));
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int b = 0; b < kXB; ++b)
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    load_lds16(xsrc[i][h] + k + b * kXHalf,
+                               reinterpret_cast<uint16_t *>(st + (FN + i * kXB + b) * 2048 + h * 1024));
+    };
+    auto chunk_at = [&](const unsigned char *block, int chunk) {
+        return block + l16 * 128 + 16 * (chunk ^ ((l16 >> 1) & 7));
+    };
+    auto fetch = [&](Frags &f, int slot) {
+        const unsigned char *st = stage_of(slot);
+        auto get = [&](auto &raw, const unsigned char *blocks, int u) { // fragment u of a row of blocks
+            using R = std::remove_reference_t<decltype(raw)>;
+            if constexpr (std::is_same_v<R, Raw8<float>>) {
+                raw.v[0] = *reinterpret_cast<const f32x4 *>(chunk_at(blocks + u * 2048, 2 * quad));
+                raw.v[1] = *reinterpret_cast<const f32x4 *>(chunk_at(blocks + u * 2048, 2 * quad + 1));
+            } else {
+                raw.v = *reinterpret_cast<const u32x4 *>(chunk_at(blocks, 4 * u + quad));
+            }
+        };
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+                get(f.w[j][u], st + j * 2048, u);
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+                get(f.x[i][u], st + (FN + i * kXB) * 2048, u);
+        }
+    };
+    auto load = [&](Frags &f, int step) { // straight from global memory, k = 32 u + 8 quad of the step
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+            const int k = step * kStep + 32 * u + 8 * quad;
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+                raw8_load(f.w[j][u], w_row(16 * j + l16) + k);
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+                raw8_load(f.x[i][u], x_row(16 * i + l16) + k);
+        }
+    };
+    auto load_tail = [&](Frags &f, int step) { // the partial last step, element by element
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+            const int k = step * kStep + 32 * u + 8 * quad;
+            const int at = k < K ? k : K - 1;
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+                raw8_load_tail(f.w[j][u], w_row(16 * j + l16) + at, K - k);
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+                raw8_load_tail(f.x[i][u], x_row(16 * i + l16) + at, K - k);
+        }
+    };
+    // Two chains where one tile alone would wait for each MFMA's result.
+    constexpr int kChains = FM * FN == 1 ? 2 : 1;
+    f32x4 acc[FN][FM], acc1 = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+            acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto multiply = [&](const Frags &f) {
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+            if constexpr (kF32Mfma) { // at e, quad q supplies the e-th of its 8 k
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+#pragma unroll
+                    for (int j = 0; j < FN; ++j)
+#pragma unroll
+                        for (int i = 0; i < FM; ++i) {
+                            f32x4 &a = kChains == 2 && (e & 1) ? acc1 : acc[j][i];
+                            a = __builtin_amdgcn_mfma_f32_16x16x4f32(raw8_at(f.w[j][u], e), raw8_at(f.x[i][u], e), a,
+                                                                     0, 0, 0);
+                        }
+            } else {
+                bf16x8v x[FM];
+#pragma unroll
+                for (int i = 0; i < FM; ++i)
+                    x[i] = raw8_bf16(f.x[i][u]);
+#pragma unroll
+                for (int j = 0; j < FN; ++j)
+#pragma unroll
+                    for (int i = 0; i < FM; ++i) {
+                        f32x4 &a = kChains == 2 && u == 1 ? acc1 : acc[j][i];
+                        a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(raw8_bf16(f.w[j][u]), x[i], a, 0, 0, 0);
+                    }
+            }
+        }
+    };
+
+    // This wave's steps: wave, wave + kWaves, ...; the partial last step goes to the next in turn.
+    const int full = K / kStep;
+    const int mine = full > wave ? (full - 1 - wave) / kWaves + 1 : 0;
+    const bool has_tail = K % kStep != 0 && full % kWaves == wave;
+    if constexpr (kStaged) {
+        // The stages are the wave's own: it waits for its loads of a stage (vmcnt: those of the younger
+        // stages stay in flight), reads the fragments, waits for the reads (lgkmcnt) and reloads it.
+        auto wait_loads = [&](auto younger) {
+            constexpr int n = decltype(younger)::value * kLoads;
+            static_assert(n < 64, "vmcnt holds 6 bits");
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_waitcnt(kWaitVmcnt0Only | (n & 15) | ((n >> 4) << 14));
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        auto wait_reads = [] {
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_waitcnt(0xC07F); // lgkmcnt(0)
+            __builtin_amdgcn_sched_barrier(0);
+        };
+#pragma unroll
+        for (int d = 0; d < kDepth; ++d)
+            if (d < mine)
+                stage(d, wave + d * kWaves);
+        int i = 0, slot = 0;
+        for (; i + kDepth < mine; ++i) {
+            Frags f;
+            wait_loads(std::integral_constant<int, kDepth - 1>{});
+            fetch(f, slot);
+            wait_reads();
+            stage(slot, wave + (i + kDepth) * kWaves);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(f);
+            slot = slot + 1 == kDepth ? 0 : slot + 1;
+        }
+        for (; i < mine; ++i) { // the last kDepth steps: nothing more to load
+            Frags f;
+            const int younger = mine - 1 - i;
+            if (kDepth > 3 && younger == 3)
+                wait_loads(std::integral_constant<int, (kDepth > 3 ? 3 : 0)>{});
+            else if (kDepth > 2 && younger == 2)
+                wait_loads(std::integral_constant<int, (kDepth > 2 ? 2 : 0)>{});
+            else if (kDepth > 1 && younger == 1)
+                wait_loads(std::integral_constant<int, (kDepth > 1 ? 1 : 0)>{});
+            else
+                wait_loads(std::integral_constant<int, 0>{});
+            fetch(f, slot);
+            multiply(f);
+            slot = slot + 1 == kDepth ? 0 : slot + 1;
+        }
+    } else {
+        Frags f[2];
+        if (mine > 0)
+            load(f[0], wave);
+        for (int i = 0; i < mine; i += 2) {
+            if (i + 1 < mine)
+                load(f[1], wave + (i + 1) * kWaves);
+            multiply(f[0]);
+            if (i + 2 < mine)
+                load(f[0], wave + (i + 2) * kWaves);
+            if (i + 1 < mine)
+                multiply(f[1]);
+        }
+    }
+    if (has_tail) {
+        Frags f;
+        load_tail(f, full);
+        multiply(f);
+    }
+    if constexpr (kChains == 2)
+        acc[0][0] = acc[0][0] + acc1;
+    // Sum over the waves in wave order; item (j, i, lane) holds columns 4 quad .. + 3 of row l16.
+    f32x4 *red = reinterpret_cast<f32x4 *>(lds);
+    if constexpr (kStaged)
+        __syncthreads(); // every wave is done with its stages
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+            red[wave * kItems + (j * FM + i) * kWaveSize + lane] = acc[j][i];
+    __syncthreads();
+    const bool wide = N % 4 == 0 && (reinterpret_cast<uintptr_t>(C) & 15u) == 0;
+    for (int item = threadIdx.x; item < kItems; item += S::kThreads) {
+        f32x4 sum = red[item];
+#pragma unroll
+        for (int w = 1; w < kWaves; ++w)
+            sum = sum + red[w * kItems + item];
+        const int tile = item / kWaveSize, j = tile / FM, i = tile % FM;
+        const int m = m0 + 16 * i + item % 16, n = n0 + 16 * j + 4 * (item % kWaveSize / 16);
+        if (m >= M || n >= N)
+            continue;
+        f32x4 v;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            v[r] = epi(sum[r] + (bias != nullptr && n + r < N ? bias[n + r] : 0.f));
+        if constexpr (kStore == GemmStore::swiglu || kStore == GemmStore::swiglu_bf16) { // N is even
+#pragma unroll
+            for (int r = 0; r < 4; r += 2) {
+                if (n + r >= N)
+                    break;
+                const float y = v[r] / (1.f + expf(-v[r])) * v[r + 1];
+                const int64_t at = int64_t(m) * (N / 2) + (n + r) / 2;
+                if constexpr (kStore == GemmStore::swiglu)
+                    C[at] = y;
+                else
+                    reinterpret_cast<uint16_t *>(C)[at] = float_to_bf16_rne(y);
+            }
+        } else {
+            static_assert(kStore != GemmStore::partial, "K is split inside the workgroup");
+            float *dst = C + int64_t(m) * N + n;
+            if (wide) {
+                f32x4 *d4 = reinterpret_cast<f32x4 *>(dst);
+                *d4 = kStore == GemmStore::residual ? *d4 + v : v;
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (n + r < N)
+                        dst[r] = kStore == GemmStore::residual ? dst[r] + v[r] : v[r];
+            }
+        }
+    }
+}
+
+// Whether few-row products take this kernel: the tiled kernels' M padding costs more than its extra
+// reads of X up to 64 rows (N = 8192, K = 2048, fp32: 25 us against 157; at 100 rows 47).
+constexpr int kRowsMax = 64;
+inline bool gemm_rows_use(int M, int K) { return M <= kRowsMax && K > 0; }
+
+// C (per kStore) = epi(X[M][K] W[N][K]^T + bias). The largest tile that fits the rows and still gives
+// every CU a workgroup: it reads X from L2 the fewest times; below that, 16 x 16 tiles, for the most
+// workgroups. (fp32 weights, M <= 16, 8192 columns: 16 x 16 tiles 14.4 us on 512 workgroups, 16 x 32
+// 18.5 on 256, so there only bf16 weights, half the bytes per tile, take the wide tile: 11.4 against
+// 13.8.)
+template <bool kRound, typename Epi, GemmStore kStore, typename TX, typename TW>
+void gemm_rows_launch(const TX *X, const TW *W, const float *bias, float *C, int M, int N, int K, Epi epi,
+                      hipStream_t stream) {
+    auto run = [&](auto shape, auto staged) {
+        using S = decltype(shape);
+        const dim3 grid(static_cast<unsigned>(blocks_for64(N, 16 * S::FN)),
+                        static_cast<unsigned>(blocks_for64(M, 16 * S::FM)));
+        launch_async(stream, gemm_rows_kernel<S, TX, TW, kRound, decltype(staged)::value, Epi, kStore>, grid,
+                     S::kThreads, X, W, bias, C, M, N, K, epi);
+    };
+    using Small = RowsShape<1, 1, 8, 2>;
+    constexpr int kAlign = 16 / sizeof(TW); // elements of X are as wide as W's, or wider
+    if (!aligned16(X) || !aligned16(W) || K % kAlign != 0) {
+        run(Small{}, std::false_type{});
+        return;
+    }
+    const int cus = cu_count();
+    auto fills = [&](int fm, int fn) { return blocks_for64(M, 16 * fm) * blocks_for64(N, 16 * fn) >= cus; };
+    if (M > 32 && fills(4, 2))
+        run(RowsShape<4, 2, 4, 2>{}, std::true_type{});
+    else if (M > 16 && fills(2, 2))
+        run(RowsShape<2, 2, 4, 3>{}, std::true_type{});
+    else if ((M > 16 || !std::is_same_v<TW, float>) && fills(1, 2))
+        run(RowsShape<1, 2, 8, 2>{}, std::true_type{});
+    else
+        run(Small{}, std::true_type{});
+}
+
+} // namespace opworks::detail

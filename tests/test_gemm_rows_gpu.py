@@ -1,0 +1,94 @@
+"""The few-row GEMM (ops/gemm_rows.hpp, up to 64 rows with weights in [out][in]): edges of its 16-row and
+16- or 32-column tiles, K around its steps of 128 bytes per row (shorter than a step, fewer steps than
+waves, a partial last step), rows that are not 16-byte aligned, and every operand type.
+
+Tolerance: products of fp32 inputs are rounded once and products of bf16 inputs are exact; a sum of K
+terms in fp32 in any order is within (K + 1) 2^-23 of sum |x w| (2^-23: the matrix core may truncate)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+FORMS = ["f32", "wbf16", "bf16", "bf16_bf16"]
+
+
+def _bf16(a):
+    """Nearest-even bf16 bits of an fp32 array, and the values they hold."""
+    u = np.ascontiguousarray(a, np.float32).view(np.uint32)
+    b = ((u.astype(np.uint64) + 0x7FFF + ((u >> 16) & 1)) >> 16).astype(np.uint16)
+    return b, (b.astype(np.uint32) << 16).view(np.float32)
+
+
+def _call(ow, form, x, w, bias, act, shift=0):
+    """Runs the entry point of `form`, its operands `shift` elements into their buffers; (result, x64, w64)."""
+    rows, k = x.shape
+    n = w.shape[0]
+    wb, wv = _bf16(w) if form != "f32" else (w, w)
+    xb, xv = _bf16(x) if form in ("bf16", "bf16_bf16") else (x, x)
+    x_in = xb if form == "bf16_bf16" else x
+
+    def up(a):
+        return ow.DeviceBuffer.from_host(np.concatenate([np.zeros(shift, a.dtype), a.reshape(-1)])).offset(shift)
+
+    dx, dw, out = up(x_in), up(wb), ow.DeviceBuffer.from_host(np.full(rows * n + shift, 7, np.float32)).offset(shift)
+    db = up(bias) if bias is not None else None
+    if form == "f32":
+        ow.ops.mat_mul_fused(dx, dw, db, out, rows, k, n, True, act)
+    elif form == "wbf16":
+        ow.ops.linear_wbf16(dx, dw, out, rows, k, n)
+    else:
+        ow.ops.linear_bf16(dx, dw, db, out, rows, k, n, act, x_bf16=form == "bf16_bf16")
+    return out.to_host().reshape(rows, n), xv.astype(np.float64), wv.astype(np.float64)
+
+
+def _check(got, x64, w64, bias, act):
+    want = x64 @ w64.T + (0 if bias is None else bias.astype(np.float64))
+    bound = (x64.shape[1] + 2) * 2.0 ** -23 * (np.abs(x64) @ np.abs(w64).T + (0 if bias is None else np.abs(bias)))
+    if act == "relu":
+        want = np.maximum(want, 0)
+    assert np.all(np.abs(got - want) <= bound + 1e-30), float(np.max(np.abs(got - want) / (bound + 1e-30)))
+
+
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("rows,n,k", [
+    (2, 16, 1), (2, 1, 40), (15, 17, 31), (16, 48, 32), (17, 33, 64), (32, 40, 72), (33, 513, 264), (64, 31, 1032),
+    (3, 100, 2048), (5, 8200, 96),                      # 8200 columns: 16 x 32 tiles for bf16 weights
+    (31, 4128, 128), (64, 4104, 200), (63, 8208, 520),  # 32 x 32 and 64 x 32 tiles, with partial tiles
+    (9, 64, 8192), (2, 20, 16640)])
+def test_rows_match_float64(ow, form, rows, n, k):
+    rng = np.random.default_rng(rows * 100003 + n * 101 + k)
+    x = rng.standard_normal((rows, k), np.float32)
+    w = rng.standard_normal((n, k), np.float32)
+    act = "none" if form == "wbf16" else "relu"
+    bias = None if form == "wbf16" else rng.uniform(-1, 1, n).astype(np.float32)
+    got, x64, w64 = _call(ow, form, x, w, bias, act)
+    _check(got, x64, w64, bias, act)
+
+
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("rows,n,k,shift", [(2, 5, 3, 0), (16, 33, 65, 0), (40, 50, 1001, 0), (8, 64, 256, 1),
+                                            (64, 20, 200, 3)])
+def test_rows_unaligned(ow, form, rows, n, k, shift):
+    """An inner dimension, or operands, that leave rows off the 16-byte grid."""
+    rng = np.random.default_rng(k + shift)
+    x = rng.standard_normal((rows, k), np.float32)
+    w = rng.standard_normal((n, k), np.float32)
+    got, x64, w64 = _call(ow, form, x, w, None, "none", shift)
+    _check(got, x64, w64, None, "none")
+
+
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("k", [96, 257])
+def test_rows_keep_infinities_to_their_outputs(ow, form, k):
+    """An infinite input or weight reaches the outputs of its row or column only, with the sign of the
+    product; rows past the last one and the K tail are padding that must not add NaNs."""
+    rng = np.random.default_rng(k)
+    x = rng.uniform(0.5, 1.5, (18, k)).astype(np.float32)
+    w = rng.uniform(0.5, 1.5, (21, k)).astype(np.float32)
+    x[17, k - 1] = np.inf
+    w[20, 3] = -np.inf
+    got, x64, w64 = _call(ow, form, x, w, None, "none")
+    want = x64 @ w64.T
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isposinf(got), np.isposinf(want))
+    assert np.array_equal(np.isneginf(got), np.isneginf(want))
+    _check(got[:17, :20], x64[:17], w64[:20], None, "none")
