@@ -5,6 +5,7 @@
 // out = (x - mean) * rstd * gamma + beta. Two-pass statistics over the
 // register-resident row (one HBM read, one write).
 
+#include "rows_split.hpp"
 #include "rowwise_kernels.hpp"
 
 namespace opworks::detail {
@@ -15,21 +16,25 @@ namespace opworks::detail {
 // and beta in LDS once per workgroup, so the output loop does not hold every gamma/beta pack
 // in registers at once (which had spilled 5 registers to scratch at that limit, +16% HBM
 // traffic), and the workgroup's rows share one read of them.
-template <int kW, int kV, bool kExact>
-__global__ __launch_bounds__(RowShape<kW>::kBlock) __attribute__((amdgpu_waves_per_eu(kV <= 8 ? 8 : 1)))
+template <int kW, int kV, RowFit kFit>
+__global__ __launch_bounds__(RowShape<kW>::kBlock) __attribute__((amdgpu_waves_per_eu(kV > 8 ? 1 : kFit == RowFit::ragged ? 7 : 8)))
 void layer_norm_reg_kernel(
     const float *__restrict__ in, float *__restrict__ out, const float *__restrict__ gamma,
     const float *__restrict__ beta, int rows, int cols, float eps) {
     const RowPos p = row_position<kW>(rows);
-    const int n4 = cols / 4;
+    constexpr bool kRagged = kFit == RowFit::ragged;
+    const int n4 = row_packs<kFit>(cols);
     const f32x4 *src = reinterpret_cast<const f32x4 *>(in + p.row * cols);
     f32x4 x[kV];
     float local = 0.f;
 #pragma unroll
     for (int k = 0; k < kV; ++k) {
         const int q = pack_index<kW>(p, k);
-        if (p.active && (kExact || q < n4)) {
-            x[k] = __builtin_nontemporal_load(src + q);
+        if (p.active && pack_valid<kW, kFit>(p, k, n4)) {
+            if constexpr (kRagged)
+                x[k] = row_pack_load(in + p.row * cols, 4 * int64_t(q), cols, 0.f);
+            else
+                x[k] = __builtin_nontemporal_load(src + q);
             local += (x[k][0] + x[k][1]) + (x[k][2] + x[k][3]);
         }
     }
@@ -39,8 +44,8 @@ void layer_norm_reg_kernel(
     __shared__ f32x4 gs[kStaged ? kV * kWaveSize : 1], bs[kStaged ? kV * kWaveSize : 1];
     if constexpr (kStaged) {
         for (int i = threadIdx.x; i < n4; i += RowShape<kW>::kBlock) {
-            gs[i] = g4[i];
-            bs[i] = b4[i];
+            gs[i] = kRagged ? row_pack_load(gamma, 4 * int64_t(i), cols, 0.f) : g4[i];
+            bs[i] = kRagged ? row_pack_load(beta, 4 * int64_t(i), cols, 0.f) : b4[i];
         }
     }
     const float mean = row_combine<kW>(wave::sum(local), p, wave::Add{}) / cols;
@@ -48,10 +53,10 @@ void layer_norm_reg_kernel(
 #pragma unroll
     for (int k = 0; k < kV; ++k) {
         const int q = pack_index<kW>(p, k);
-        if (p.active && (kExact || q < n4)) {
+        if (p.active && pack_valid<kW, kFit>(p, k, n4)) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const float d = x[k][j] - mean;
+                const float d = kRagged && 4 * q + j >= cols ? 0.f : x[k][j] - mean;
                 local = fmaf(d, d, local);
             }
         }
@@ -63,13 +68,26 @@ void layer_norm_reg_kernel(
 #pragma unroll
     for (int k = 0; k < kV; ++k) {
         const int q = pack_index<kW>(p, k);
-        if (p.active && (kExact || q < n4)) {
-            const f32x4 g = kStaged ? gs[q] : g4[q], b = kStaged ? bs[q] : b4[q];
+        if (p.active && pack_valid<kW, kFit>(p, k, n4)) {
+            f32x4 g, b;
+            if constexpr (kStaged) {
+                g = gs[q];
+                b = bs[q];
+            } else if constexpr (kRagged) {
+                g = row_pack_load(gamma, 4 * int64_t(q), cols, 0.f);
+                b = row_pack_load(beta, 4 * int64_t(q), cols, 0.f);
+            } else {
+                g = g4[q];
+                b = b4[q];
+            }
             f32x4 r;
 #pragma unroll
             for (int j = 0; j < 4; ++j)
                 r[j] = fmaf((x[k][j] - mean) * rstd, g[j], b[j]);
-            __builtin_nontemporal_store(r, dst + q);
+            if constexpr (kRagged)
+                row_pack_store(out + p.row * cols, 4 * int64_t(q), cols, r);
+            else
+                __builtin_nontemporal_store(r, dst + q);
         }
         if constexpr (!kStaged)
             __builtin_amdgcn_sched_barrier(0); // keep each pack's gamma/beta loads beside their use
@@ -107,17 +125,22 @@ inline void layer_norm(const float *in, float *out, const float *gamma, const fl
     detail::require(in && out && gamma && beta, "layer norm requires non-null pointers");
     const bool packed = detail::aligned16(in) && detail::aligned16(out) && detail::aligned16(gamma) &&
                         detail::aligned16(beta);
-    const detail::RowPlan plan = detail::plan_row(cols, packed);
+    const detail::RowPlan plan = detail::plan_row(cols);
+    if (plan.waves == 0 && detail::row_split_ok(in, out, rows, cols)) {
+        detail::row_split_launch<detail::LayerNormSplit>(in, out, gamma, beta, rows, cols, eps, stream);
+        return;
+    }
     if (plan.waves == 0) {
         launch_async(stream, detail::layer_norm_stream_kernel, rows, kThreads, in, out, gamma, beta, cols, eps);
         return;
     }
     detail::dispatch_row_plan(plan, [&](auto w, auto v) {
         constexpr int kW = decltype(w)::value, kV = decltype(v)::value;
-        auto *kernel = detail::row_plan_exact<kW, kV>(cols) ? detail::layer_norm_reg_kernel<kW, kV, true>
-                                                              : detail::layer_norm_reg_kernel<kW, kV, false>;
-        launch_async(stream, kernel, detail::row_grid<kW>(rows),
-                     detail::RowShape<kW>::kBlock, in, out, gamma, beta, rows, cols, eps);
+        detail::dispatch_row_fit(detail::row_fit<kW, kV>(cols, packed), [&](auto fit) {
+            launch_async(stream, detail::layer_norm_reg_kernel<kW, kV, decltype(fit)::value>,
+                         detail::row_grid<kW>(rows), detail::RowShape<kW>::kBlock, in, out, gamma, beta, rows, cols,
+                         eps);
+        });
     });
 }
 

@@ -4,27 +4,33 @@
 // Per row: ss = sum(x^2); inv = rsqrtf(ss/cols + eps); out = x * inv * weight.
 
 #include "../core/bf16.hpp"
+#include "rows_split.hpp"
 #include "rowwise_kernels.hpp"
 
 namespace opworks::detail {
 
 // OT = float, or uint16_t: the output rounded to bf16 (nearest-even) as it is stored, for a
 // bf16 GEMM that would round it on load anyway (the same bits, half the bytes, no extra pass).
-template <int kW, int kV, bool kExact, typename OT = float>
+template <int kW, int kV, RowFit kFit, typename OT = float>
 __global__ __launch_bounds__(RowShape<kW>::kBlock) void rms_norm_reg_kernel(const float *__restrict__ x,
                                                                              const float *__restrict__ weight,
                                                                              OT *__restrict__ out, int rows,
                                                                              int cols, float eps) {
     const RowPos p = row_position<kW>(rows);
-    const int n4 = cols / 4;
+    constexpr bool kRagged = kFit == RowFit::ragged;
+    static_assert(!kRagged || std::is_same_v<OT, float>, "bf16 output takes aligned rows");
+    const int n4 = row_packs<kFit>(cols);
     const f32x4 *src = reinterpret_cast<const f32x4 *>(x + p.row * cols);
     f32x4 v[kV];
     float local = 0.f;
 #pragma unroll
     for (int k = 0; k < kV; ++k) {
         const int q = pack_index<kW>(p, k);
-        if (p.active && (kExact || q < n4)) {
-            v[k] = __builtin_nontemporal_load(src + q);
+        if (p.active && pack_valid<kW, kFit>(p, k, n4)) {
+            if constexpr (kRagged)
+                v[k] = row_pack_load(x + p.row * cols, 4 * int64_t(q), cols, 0.f);
+            else
+                v[k] = __builtin_nontemporal_load(src + q);
 #pragma unroll
             for (int j = 0; j < 4; ++j)
                 local = fmaf(v[k][j], v[k][j], local);
@@ -35,13 +41,19 @@ __global__ __launch_bounds__(RowShape<kW>::kBlock) void rms_norm_reg_kernel(cons
 #pragma unroll
     for (int k = 0; k < kV; ++k) {
         const int q = pack_index<kW>(p, k);
-        if (p.active && (kExact || q < n4)) {
-            const f32x4 w = w4[q];
+        if (p.active && pack_valid<kW, kFit>(p, k, n4)) {
+            f32x4 w;
+            if constexpr (kRagged)
+                w = row_pack_load(weight, 4 * int64_t(q), cols, 0.f);
+            else
+                w = w4[q];
             f32x4 r;
 #pragma unroll
             for (int j = 0; j < 4; ++j)
                 r[j] = v[k][j] * inv * w[j];
-            if constexpr (std::is_same_v<OT, float>) {
+            if constexpr (kRagged) {
+                row_pack_store(out + p.row * cols, 4 * int64_t(q), cols, r);
+            } else if constexpr (std::is_same_v<OT, float>) {
                 __builtin_nontemporal_store(r, reinterpret_cast<f32x4 *>(out + p.row * cols) + q);
             } else {
                 const uint2 b = make_uint2(uint32_t(float_to_bf16_rne(r[0])) | (uint32_t(float_to_bf16_rne(r[1])) << 16),
@@ -80,17 +92,21 @@ inline void rms_norm(const float *x, const float *weight, float *out, int rows, 
     detail::require(x && weight && out, "rms_norm requires non-null pointers");
     detail::require(eps > 0.f, "rms_norm epsilon must be positive");
     const bool packed = detail::aligned16(x) && detail::aligned16(weight) && detail::aligned16(out);
-    const detail::RowPlan plan = detail::plan_row_for_rows(rows, cols, packed);
+    const detail::RowPlan plan = detail::plan_row_for_rows(rows, cols);
+    if (plan.waves == 0 && detail::row_split_ok(x, out, rows, cols)) {
+        detail::row_split_launch<detail::RmsNormSplit>(x, out, weight, nullptr, rows, cols, eps, stream);
+        return;
+    }
     if (plan.waves == 0) {
         launch_async(stream, detail::rms_norm_stream_kernel, rows, kThreads, x, weight, out, cols, eps);
         return;
     }
     detail::dispatch_row_plan_for_rows(plan, [&](auto w, auto v) {
         constexpr int kW = decltype(w)::value, kV = decltype(v)::value;
-        auto *kernel = detail::row_plan_exact<kW, kV>(cols) ? detail::rms_norm_reg_kernel<kW, kV, true>
-                                                              : detail::rms_norm_reg_kernel<kW, kV, false>;
-        launch_async(stream, kernel, detail::row_grid<kW>(rows),
-                     detail::RowShape<kW>::kBlock, x, weight, out, rows, cols, eps);
+        detail::dispatch_row_fit(detail::row_fit<kW, kV>(cols, packed), [&](auto fit) {
+            launch_async(stream, detail::rms_norm_reg_kernel<kW, kV, decltype(fit)::value>, detail::row_grid<kW>(rows),
+                         detail::RowShape<kW>::kBlock, x, weight, out, rows, cols, eps);
+        });
     });
 }
 
@@ -154,8 +170,9 @@ __global__ __launch_bounds__(RowShape<kW>::kBlock) void splitk_residual_rms_norm
 
 // True when splitk_residual_rms_norm can run on this shape (an exact register plan, aligned rows).
 inline bool splitk_residual_rms_norm_ok(int rows, int cols, const void *hidden, const void *weight, const void *out) {
-    const RowPlan plan = plan_row_for_rows(rows, cols, aligned16(hidden) && aligned16(weight) && aligned16(out));
-    return plan.waves != 0 && cols / 4 == plan.waves * plan.packs * kWaveSize;
+    const RowPlan plan = plan_row_for_rows(rows, cols);
+    return aligned16(hidden) && aligned16(weight) && aligned16(out) && plan.waves != 0 && cols % 4 == 0 &&
+           cols / 4 == plan.waves * plan.packs * kWaveSize;
 }
 
 template <typename OT>
@@ -163,7 +180,7 @@ inline void splitk_residual_rms_norm(const float *part, int splits, float *hidde
                                      int rows, int cols, float eps, hipStream_t stream) {
     require(splitk_residual_rms_norm_ok(rows, cols, hidden, weight, out) && splits >= 1 && eps > 0.f,
             "splitk_residual_rms_norm: unsupported shape");
-    const RowPlan plan = plan_row_for_rows(rows, cols, true);
+    const RowPlan plan = plan_row_for_rows(rows, cols);
     dispatch_row_plan_for_rows(plan, [&](auto w, auto v) {
         constexpr int kW = decltype(w)::value, kV = decltype(v)::value;
         launch_async(stream, splitk_residual_rms_norm_kernel<kW, kV, OT>, row_grid<kW>(rows), RowShape<kW>::kBlock,
@@ -179,12 +196,13 @@ inline void rms_norm_to_bf16(const float *x, const float *weight, uint16_t *out,
     if (rows == 0)
         return;
     require(x && weight && out && eps > 0.f, "rms_norm_to_bf16: bad arguments");
-    const RowPlan plan = plan_row_for_rows(rows, cols, aligned16(x) && aligned16(weight) && aligned16(out));
-    require(plan.waves != 0, "rms_norm_to_bf16 needs aligned rows of a multiple of 4 columns");
+    const RowPlan plan = plan_row_for_rows(rows, cols);
+    require(plan.waves != 0 && cols % 4 == 0 && aligned16(x) && aligned16(weight) && aligned16(out), "rms_norm_to_bf16 needs aligned rows of a multiple of 4 columns");
     dispatch_row_plan_for_rows(plan, [&](auto w, auto v) {
         constexpr int kW = decltype(w)::value, kV = decltype(v)::value;
-        auto *kernel = row_plan_exact<kW, kV>(cols) ? rms_norm_reg_kernel<kW, kV, true, uint16_t>
-                                                     : rms_norm_reg_kernel<kW, kV, false, uint16_t>;
+        auto *kernel = row_fit<kW, kV>(cols, true) == RowFit::exact
+                           ? rms_norm_reg_kernel<kW, kV, RowFit::exact, uint16_t>
+                           : rms_norm_reg_kernel<kW, kV, RowFit::bounded, uint16_t>;
         launch_async(stream, kernel, row_grid<kW>(rows), RowShape<kW>::kBlock, x, weight, out, rows, cols, eps);
     });
 }

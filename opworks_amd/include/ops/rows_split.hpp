@@ -1,0 +1,217 @@
+#pragma once
+
+// Row ops (softmax, layer_norm, rms_norm) on rows too long for one workgroup's registers.
+//
+// One workgroup per row leaves most of the GPU idle when there are few such rows (32 rows of a
+// 128256-token vocabulary: 32 of 256 CUs) and re-reads the row for every pass. Here a row is cut
+// into chunks of at most 4 * kV * 256 elements, one workgroup each, in two launches:
+//  1. row_split_stats_kernel: each chunk is read once into registers and reduced to two floats;
+//  2. row_split_apply_kernel: each chunk's workgroup combines the row's statistics in chunk order,
+//     then maps its chunk. The second read comes from the caches up to their size.
+// There is no workspace: the statistics travel in the output. A chunk's workgroup writes its two
+// floats into the start of every chunk of its output row, so the second launch reads them from the
+// range that its own workgroup then overwrites, and no workgroup touches a range that another still
+// reads. That needs an output apart from the input (row_split_ok); 2 * chunks <= a chunk's length.
+// The result depends only on the row and its length.
+//
+// Softmax 32 x 128256 (16.4 MB each way): 314 us on one 256-lane workgroup per row -> 13.0.
+
+#include <cstdint>
+
+#include "rowwise_kernels.hpp"
+
+namespace opworks::detail {
+
+constexpr int kSplitThreads = 256;
+
+// First element of chunk c of `chunks`; chunk boundaries are whole packs of 4 from the row's start.
+__device__ __forceinline__ int64_t row_split_begin(int cols, int chunks, int c) {
+    return c == chunks ? cols : 4 * (int64_t(cols / 4) * c / chunks);
+}
+
+// This thread's packs of [begin, end): pack p at begin + 4 (threadIdx.x + 256 p), `fill` past the end.
+template <int kV>
+__device__ __forceinline__ void row_split_load(const float *row, int64_t begin, int64_t end, float fill,
+                                               f32x4 (&x)[kV]) {
+#pragma unroll
+    for (int p = 0; p < kV; ++p) {
+        const int64_t at = begin + 4 * (int64_t(threadIdx.x) + kSplitThreads * p);
+        x[p] = row_pack_load(row, at, end, fill);
+    }
+}
+
+// Statistics policies: partial() reduces a chunk (all lanes get both floats), Combined accumulates the
+// row's partials per lane and finish() reduces them over the workgroup, apply() maps one element.
+struct SoftmaxSplit {
+    static constexpr bool kParams = false;
+    static constexpr float kFill = kNegInf;
+    template <int kV> __device__ static float2 partial(const f32x4 (&x)[kV], int64_t, int64_t) {
+        float m = kNegInf;
+#pragma unroll
+        for (int p = 0; p < kV; ++p)
+            m = fmaxf(m, fmaxf(fmaxf(x[p][0], x[p][1]), fmaxf(x[p][2], x[p][3])));
+        m = block_reduce_all<ReduceMax>(m);
+        const float ref = m == kNegInf ? 0.f : m; // a chunk of -inf only (or NaN) sums to 0 (or NaN)
+        float s = 0.f;
+#pragma unroll
+        for (int p = 0; p < kV; ++p)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                s += expf(x[p][j] - ref);
+        return {m, block_reduce_all<ReduceSum>(s)};
+    }
+    __device__ static float2 combine(const float *part, int chunks, int) { // {m, 1 / s} of the row
+        float m = kNegInf;
+        for (int c = threadIdx.x; c < chunks; c += kSplitThreads)
+            m = fmaxf(m, part[2 * c]);
+        m = block_reduce_all<ReduceMax>(m);
+        float s = 0.f;
+        for (int c = threadIdx.x; c < chunks; c += kSplitThreads)
+            s = fmaf(part[2 * c + 1], expf(part[2 * c] - m), s); // every element -inf: NaN, as one pass gives
+        return {m, 1.f / block_reduce_all<ReduceSum>(s)};
+    }
+    __device__ static float apply(float x, const float2 &st, float, float, float) { return expf(x - st.x) * st.y; }
+};
+
+struct LayerNormSplit {
+    static constexpr bool kParams = true;
+    static constexpr float kFill = 0.f;
+    // {mean, sum of squared distances to it} of the chunk
+    template <int kV> __device__ static float2 partial(const f32x4 (&x)[kV], int64_t begin, int64_t end) {
+        float s = 0.f;
+#pragma unroll
+        for (int p = 0; p < kV; ++p)
+            s += (x[p][0] + x[p][1]) + (x[p][2] + x[p][3]);
+        const float mean = block_reduce_all<ReduceSum>(s) / static_cast<float>(end - begin);
+        float ss = 0.f;
+#pragma unroll
+        for (int p = 0; p < kV; ++p) {
+            const int64_t at = begin + 4 * (int64_t(threadIdx.x) + kSplitThreads * p);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const float d = at + j < end ? x[p][j] - mean : 0.f;
+                ss = fmaf(d, d, ss);
+            }
+        }
+        return {mean, block_reduce_all<ReduceSum>(ss)};
+    }
+    __device__ static float2 combine(const float *part, int chunks, int cols) { // {mean, variance} of the row
+        float s = 0.f;
+        for (int c = threadIdx.x; c < chunks; c += kSplitThreads)
+            s = fmaf(part[2 * c], chunk_len(cols, chunks, c), s);
+        const float mean = block_reduce_all<ReduceSum>(s) / cols;
+        float ss = 0.f;
+        for (int c = threadIdx.x; c < chunks; c += kSplitThreads) {
+            const float d = part[2 * c] - mean;
+            ss += fmaf(d * d, chunk_len(cols, chunks, c), part[2 * c + 1]);
+        }
+        return {mean, block_reduce_all<ReduceSum>(ss) / cols};
+    }
+    __device__ static float2 with_eps(const float2 &st, float eps) { return {st.x, rsqrtf(st.y + eps)}; }
+    __device__ static float apply(float x, const float2 &st, float, float gamma, float beta) {
+        return fmaf((x - st.x) * st.y, gamma, beta);
+    }
+
+  private:
+    __device__ static float chunk_len(int cols, int chunks, int c) {
+        return static_cast<float>(row_split_begin(cols, chunks, c + 1) - row_split_begin(cols, chunks, c));
+    }
+};
+
+struct RmsNormSplit {
+    static constexpr bool kParams = true;
+    static constexpr float kFill = 0.f;
+    template <int kV> __device__ static float2 partial(const f32x4 (&x)[kV], int64_t, int64_t) {
+        float ss = 0.f;
+#pragma unroll
+        for (int p = 0; p < kV; ++p)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                ss = fmaf(x[p][j], x[p][j], ss);
+        return {block_reduce_all<ReduceSum>(ss), 0.f};
+    }
+    __device__ static float2 combine(const float *part, int chunks, int cols) { // {0, mean square} of the row
+        float ss = 0.f;
+        for (int c = threadIdx.x; c < chunks; c += kSplitThreads)
+            ss += part[2 * c];
+        return {0.f, block_reduce_all<ReduceSum>(ss) / cols};
+    }
+    __device__ static float2 with_eps(const float2 &st, float eps) { return {st.x, rsqrtf(st.y + eps)}; }
+    __device__ static float apply(float x, const float2 &st, float, float gamma, float) { return x * st.y * gamma; }
+};
+
+template <typename Op, int kV>
+__global__ __launch_bounds__(kSplitThreads) void row_split_stats_kernel(const float *__restrict__ in,
+                                                                        float *__restrict__ out, int cols, int chunks) {
+    const int c = blockIdx.x % chunks;
+    const int64_t row = blockIdx.x / chunks;
+    const int64_t begin = row_split_begin(cols, chunks, c), end = row_split_begin(cols, chunks, c + 1);
+    f32x4 x[kV];
+    row_split_load<kV>(in + row * cols, begin, end, Op::kFill, x);
+    const float2 st = Op::template partial<kV>(x, begin, end);
+    for (int d = threadIdx.x; d < chunks; d += kSplitThreads) { // one copy for every chunk of the row
+        float *slot = out + row * cols + row_split_begin(cols, chunks, d) + 2 * c;
+        slot[0] = st.x;
+        slot[1] = st.y;
+    }
+}
+
+// Reads the statistics at the start of its own output chunk, then overwrites them: every lane has
+// read before the barriers of combine()'s reductions, and the stores come after them. `out` is read
+// and written, so it is not __restrict__.
+template <typename Op, int kV>
+__global__ __launch_bounds__(kSplitThreads) void row_split_apply_kernel(const float *__restrict__ in, float *out,
+                                                                        const float *__restrict__ gamma,
+                                                                        const float *__restrict__ beta, int cols,
+                                                                        int chunks, float eps) {
+    const int c = blockIdx.x % chunks;
+    const int64_t row = blockIdx.x / chunks;
+    const int64_t begin = row_split_begin(cols, chunks, c), end = row_split_begin(cols, chunks, c + 1);
+    f32x4 x[kV];
+    row_split_load<kV>(in + row * cols, begin, end, Op::kFill, x);
+    float2 st = Op::combine(out + row * cols + begin, chunks, cols);
+    if constexpr (Op::kParams)
+        st = Op::with_eps(st, eps);
+#pragma unroll
+    for (int p = 0; p < kV; ++p) {
+        const int64_t at = begin + 4 * (int64_t(threadIdx.x) + kSplitThreads * p);
+        f32x4 g = {1.f, 1.f, 1.f, 1.f}, b = {0.f, 0.f, 0.f, 0.f}, y;
+        if constexpr (Op::kParams) {
+            g = row_pack_load(gamma, at, end, 0.f);
+            if (beta != nullptr)
+                b = row_pack_load(beta, at, end, 0.f);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            y[j] = Op::apply(x[p][j], st, eps, g[j], b[j]);
+        row_pack_store(out + row * cols, at, end, y);
+    }
+}
+
+// Chunks of a row at kV packs per lane, and whether the split form takes the row: the statistics of
+// all chunks fit into each of them, and the output lies apart from the input.
+inline int row_split_chunks(int cols, int v) { return static_cast<int>(blocks_for64(cols, int64_t(4) * v * kSplitThreads - 4)); }
+inline bool row_split_ok(const float *in, const float *out, int rows, int cols) {
+    const int chunks = row_split_chunks(cols, cols <= (1 << 20) ? 4 : 16);
+    const int64_t n = int64_t(rows) * cols;
+    return cols > kRowMaxRegCols && 2 * int64_t(chunks) <= 4 * (int64_t(cols / 4) / chunks) && rows <= INT32_MAX / chunks &&
+           (in + n <= out || out + n <= in);
+}
+
+template <typename Op>
+inline void row_split_launch(const float *in, float *out, const float *gamma, const float *beta, int rows, int cols,
+                             float eps, hipStream_t stream) {
+    auto run = [&](auto v) {
+        constexpr int kV = decltype(v)::value;
+        const int chunks = row_split_chunks(cols, kV);
+        launch_async(stream, row_split_stats_kernel<Op, kV>, rows * chunks, kSplitThreads, in, out, cols, chunks);
+        launch_async(stream, row_split_apply_kernel<Op, kV>, rows * chunks, kSplitThreads, in, out, gamma, beta, cols,
+                     chunks, eps);
+    };
+    if (cols <= (1 << 20))
+        run(std::integral_constant<int, 4>{});
+    else
+        run(std::integral_constant<int, 16>{});
+}
+
+} // namespace opworks::detail

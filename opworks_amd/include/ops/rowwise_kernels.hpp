@@ -9,9 +9,11 @@
 // written once (8 bytes per element of traffic). Row statistics are reduced
 // with DPP inside each wave; rows spanning several waves exchange one partial
 // per wave through LDS and combine them in a fixed order, so every wave of the
-// row gets the identical value. Shapes the register plan cannot hold (cols not
-// a multiple of 4, misaligned rows, or more than 32768 columns) use a
-// streaming kernel that re-reads the row.
+// row gets the identical value. Rows off the 16-byte grid (cols not a multiple
+// of 4, or misaligned pointers) keep the plan on 16-byte accesses at 4-byte
+// alignment (RowFit::ragged). Rows of more than 32768 columns are cut over
+// several workgroups (rows_split.hpp); what is left (fewer than 4 columns, a
+// long row in place) uses a streaming kernel that re-reads the row.
 
 #include <cstdint>
 #include <type_traits>
@@ -53,9 +55,44 @@ template <int kW> __device__ __forceinline__ int pack_index(const RowPos &p, int
     return (k * kW + p.wave_in_row) * kWaveSize + p.lane;
 }
 
+// How a plan's packs cover a row: every pack inside it and aligned; some past its end, aligned; or
+// rows at any alignment with a partial last pack.
+enum class RowFit { exact, bounded, ragged };
+
+// Packs that hold elements of a row, the partial last one included.
+template <RowFit kFit> __device__ __forceinline__ int row_packs(int cols) {
+    return kFit == RowFit::ragged ? (cols + 3) / 4 : cols / 4;
+}
+
 // True when pack k of this lane lies inside the row (always, for exact plans).
-template <int kW, bool kExact> __device__ __forceinline__ bool pack_valid(const RowPos &p, int k, int n4) {
-    return kExact || pack_index<kW>(p, k) < n4;
+template <int kW, RowFit kFit> __device__ __forceinline__ bool pack_valid(const RowPos &p, int k, int n4) {
+    return kFit == RowFit::exact || pack_index<kW>(p, k) < n4;
+}
+
+using f32x4u = f32x4 __attribute__((aligned(4))); // 16-byte access at 4-byte alignment
+
+// Elements at .. at + 3 of a run that ends at `end` (at least 4 elements long, the run's start at
+// row[0] or later); `fill` past its end. One unconditional load: a pack that crosses the end reads the
+// run's last 4 elements and shifts them down.
+__device__ __forceinline__ f32x4 row_pack_load(const float *row, int64_t at, int64_t end, float fill) {
+    const int64_t past = at - (end - 4); // elements to shift by, if positive
+    const f32x4 v = *reinterpret_cast<const f32x4u *>(row + (past > 0 ? end - 4 : at));
+    f32x4 r;
+    r[0] = past <= 0 ? v[0] : past == 1 ? v[1] : past == 2 ? v[2] : past == 3 ? v[3] : fill;
+    r[1] = past <= 0 ? v[1] : past == 1 ? v[2] : past == 2 ? v[3] : fill;
+    r[2] = past <= 0 ? v[2] : past == 1 ? v[3] : fill;
+    r[3] = past <= 0 ? v[3] : fill;
+    return r;
+}
+__device__ __forceinline__ void row_pack_store(float *row, int64_t at, int64_t end, const f32x4 &v) {
+    if (at + 4 <= end) {
+        __builtin_nontemporal_store(v, reinterpret_cast<f32x4u *>(row + at));
+    } else {
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+            if (at + j < end)
+                row[at + j] = v[j];
+    }
 }
 
 // Loads this lane's kV packs of its row as one unpredicated batch: a wave past
@@ -65,11 +102,19 @@ template <int kW, bool kExact> __device__ __forceinline__ bool pack_valid(const 
 // vmcnt(0) wait per pack (4096 x 1024: 6.13 against 6.96 us). RMSNorm keeps
 // its predicated loads, which measured faster for its 8 packs per lane
 // (8192 x 2048: 21.4 against 22.9 us). Callers mask invalid packs with
-// pack_valid and store only for active waves.
-template <int kW, int kV, bool kExact>
+// pack_valid and store only for active waves. A ragged row's partial pack is
+// filled up with `fill`.
+template <int kW, int kV, RowFit kFit>
 __device__ __forceinline__ void load_row_packs(const float *__restrict__ in, int rows, int cols, const RowPos &p,
-                                               f32x4 (&v)[kV]) {
+                                               f32x4 (&v)[kV], float fill) {
     const int64_t row = p.active ? p.row : rows - 1;
+    if constexpr (kFit == RowFit::ragged) {
+#pragma unroll
+        for (int k = 0; k < kV; ++k)
+            v[k] = row_pack_load(in + row * cols, 4 * int64_t(pack_index<kW>(p, k)), cols, fill);
+        return;
+    }
+    constexpr bool kExact = kFit == RowFit::exact;
     const int n4 = cols / 4;
     const f32x4 *src = reinterpret_cast<const f32x4 *>(in + row * cols);
 #pragma unroll
@@ -104,10 +149,10 @@ struct RowPlan {
     int packs = 0;
 };
 
-inline RowPlan plan_row(int cols, bool packed) {
-    if (!packed || cols % 4 != 0 || cols > kRowMaxRegCols)
+inline RowPlan plan_row(int cols) {
+    if (cols < 4 || cols > kRowMaxRegCols)
         return {};
-    const int n4 = cols / 4;
+    const int n4 = (cols + 3) / 4;
     if (n4 <= 64)
         return {1, 1};
     if (n4 <= 128)
@@ -129,8 +174,8 @@ inline RowPlan plan_row(int cols, bool packed) {
 // row over more waves with fewer packs each, down to 2 packs per lane, so the GPU has enough
 // waves in flight: 512 x 2048 (a 512-token prefill's RMSNorm) runs 4 waves of 2 packs per row
 // instead of 1 wave of 8. Only the row ops whose dispatch carries these shapes use it.
-inline RowPlan plan_row_for_rows(int rows, int cols, bool packed) {
-    RowPlan p = plan_row(cols, packed);
+inline RowPlan plan_row_for_rows(int rows, int cols) {
+    RowPlan p = plan_row(cols);
     while (p.waves != 0 && p.packs >= 4 && p.waves <= 4 && int64_t(rows) * p.waves < 2048) {
         p.waves *= 2;
         p.packs /= 2;
@@ -169,10 +214,23 @@ template <typename Fn> inline void dispatch_row_plan_for_rows(const RowPlan &pla
     }
 }
 
-// True when the plan's kW * kV * 64 packs cover the row exactly: the kernels
-// then drop the per-lane bounds test, which keeps every load of a lane in one
-// unpredicated batch.
-template <int kW, int kV> inline bool row_plan_exact(int cols) { return cols / 4 == kW * kV * kWaveSize; }
+// How the plan's kW * kV * 64 packs fit the row: when they cover it exactly the kernels drop the
+// per-lane bounds test, which keeps every load of a lane in one unpredicated batch. `packed`: every
+// pointer is 16-byte aligned.
+template <int kW, int kV> inline RowFit row_fit(int cols, bool packed) {
+    if (!packed || cols % 4 != 0)
+        return RowFit::ragged;
+    return cols / 4 == kW * kV * kWaveSize ? RowFit::exact : RowFit::bounded;
+}
+
+// Calls fn(FitTag{}) with the std::integral_constant of `fit`.
+template <typename Fn> inline void dispatch_row_fit(RowFit fit, Fn &&fn) {
+    switch (fit) {
+    case RowFit::exact: fn(std::integral_constant<RowFit, RowFit::exact>{}); break;
+    case RowFit::bounded: fn(std::integral_constant<RowFit, RowFit::bounded>{}); break;
+    case RowFit::ragged: fn(std::integral_constant<RowFit, RowFit::ragged>{}); break;
+    }
+}
 
 template <int kW> inline int row_grid(int rows) {
     return static_cast<int>(blocks_for64(rows, RowShape<kW>::kRowsPerBlock));

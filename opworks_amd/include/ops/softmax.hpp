@@ -6,28 +6,29 @@
 // register-resident kernel multiplies by 1/s: within 1.5 ulp of the divide).
 // Register-resident rows compute each expf once and read the row once.
 
+#include "rows_split.hpp"
 #include "rowwise_kernels.hpp"
 
 namespace opworks::detail {
 
-template <int kW, int kV, bool kExact>
+template <int kW, int kV, RowFit kFit>
 __global__ __launch_bounds__(RowShape<kW>::kBlock) void softmax_rows_reg_kernel(const float *__restrict__ in,
                                                                                  float *__restrict__ out, int rows,
                                                                                  int cols) {
     const RowPos p = row_position<kW>(rows);
-    const int n4 = cols / 4;
+    const int n4 = row_packs<kFit>(cols);
     f32x4 x[kV];
-    load_row_packs<kW, kV, kExact>(in, rows, cols, p, x);
+    load_row_packs<kW, kV, kFit>(in, rows, cols, p, x, kNegInf);
     float local_max = kNegInf;
 #pragma unroll
     for (int k = 0; k < kV; ++k)
-        if (pack_valid<kW, kExact>(p, k, n4))
+        if (pack_valid<kW, kFit>(p, k, n4))
             local_max = fmaxf(local_max, fmaxf(fmaxf(x[k][0], x[k][1]), fmaxf(x[k][2], x[k][3])));
     const float m = row_combine<kW>(wave::max(local_max), p, wave::Max{});
     float local_sum = 0.f;
 #pragma unroll
     for (int k = 0; k < kV; ++k) {
-        if (pack_valid<kW, kExact>(p, k, n4)) {
+        if (pack_valid<kW, kFit>(p, k, n4)) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 x[k][j] = expf(x[k][j] - m);
@@ -41,12 +42,15 @@ __global__ __launch_bounds__(RowShape<kW>::kBlock) void softmax_rows_reg_kernel(
 #pragma unroll
     for (int k = 0; k < kV; ++k) {
         const int q = pack_index<kW>(p, k);
-        if (p.active && (kExact || q < n4)) {
+        if (p.active && pack_valid<kW, kFit>(p, k, n4)) {
             f32x4 r;
 #pragma unroll
             for (int j = 0; j < 4; ++j)
                 r[j] = x[k][j] * inv_s;
-            __builtin_nontemporal_store(r, dst + q);
+            if constexpr (kFit == RowFit::ragged)
+                row_pack_store(out + p.row * cols, 4 * int64_t(q), cols, r);
+            else
+                __builtin_nontemporal_store(r, dst + q);
         }
     }
 }
@@ -76,17 +80,22 @@ inline void softmax(const float *in, float *out, int rows, int cols, hipStream_t
         return;
     detail::require(cols > 0, "softmax requires positive columns for nonempty rows");
     detail::require(in && out, "softmax requires non-null pointers");
-    const detail::RowPlan plan = detail::plan_row(cols, detail::aligned16(in) && detail::aligned16(out));
+    const bool packed = detail::aligned16(in) && detail::aligned16(out);
+    const detail::RowPlan plan = detail::plan_row(cols);
+    if (plan.waves == 0 && detail::row_split_ok(in, out, rows, cols)) {
+        detail::row_split_launch<detail::SoftmaxSplit>(in, out, nullptr, nullptr, rows, cols, 0.f, stream);
+        return;
+    }
     if (plan.waves == 0) {
         launch_async(stream, detail::softmax_rows_stream_kernel, rows, kThreads, in, out, cols);
         return;
     }
     detail::dispatch_row_plan(plan, [&](auto w, auto v) {
         constexpr int kW = decltype(w)::value, kV = decltype(v)::value;
-        auto *kernel = detail::row_plan_exact<kW, kV>(cols) ? detail::softmax_rows_reg_kernel<kW, kV, true>
-                                                              : detail::softmax_rows_reg_kernel<kW, kV, false>;
-        launch_async(stream, kernel, detail::row_grid<kW>(rows),
-                     detail::RowShape<kW>::kBlock, in, out, rows, cols);
+        detail::dispatch_row_fit(detail::row_fit<kW, kV>(cols, packed), [&](auto fit) {
+            launch_async(stream, detail::softmax_rows_reg_kernel<kW, kV, decltype(fit)::value>,
+                         detail::row_grid<kW>(rows), detail::RowShape<kW>::kBlock, in, out, rows, cols);
+        });
     });
 }
 

@@ -1,0 +1,90 @@
+"""Row ops on rows beyond or off the 16-byte register plan: more than 32768 columns (cut over several
+workgroups, statistics passed through the output), column counts that are no multiple of 4, misaligned
+pointers, and both in place. Against numpy in float64.
+
+Tolerance: sums of up to 2^21 terms of one sign in fp32, tree-shaped over lanes and waves with at most
+64 terms in a chain, stay within 1e-5 relative; the framework's own bar is |a - e| <= 1e-5 (1 + |e|)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+OPS = ["softmax", "layer_norm", "rms_norm"]
+
+
+def _want(op, x, g, b):
+    x = x.astype(np.float64)
+    if op == "softmax":
+        with np.errstate(invalid="ignore"):
+            e = np.exp(x - x.max(1, keepdims=True))
+            return e / e.sum(1, keepdims=True)
+    if op == "rms_norm":
+        return x / np.sqrt((x * x).mean(1, keepdims=True) + 1e-5) * g
+    return (x - x.mean(1, keepdims=True)) / np.sqrt(x.var(1, keepdims=True) + 1e-5) * g + b
+
+
+def _run(ow, op, x, g, b, shift=0, in_place=False):
+    rows, cols = x.shape
+
+    def up(a):
+        return ow.DeviceBuffer.from_host(np.concatenate([np.zeros(shift, np.float32), a.reshape(-1)])).offset(shift)
+
+    dx, dg, db = up(x), up(g), up(b)
+    guard = np.full(4, 7, np.float32)
+    out = dx if in_place else up(np.concatenate([np.full(rows * cols, 9, np.float32), guard]))
+    if op == "softmax":
+        ow.ops.softmax(dx, out, rows, cols)
+    elif op == "layer_norm":
+        ow.ops.layer_norm(dx, out, dg, db, rows, cols, 1e-5)
+    else:
+        ow.ops.rms_norm(dx, dg, out, rows, cols, 1e-5)
+    got = out.to_host()
+    if not in_place:
+        assert np.array_equal(got[rows * cols:], guard)
+    return got[:rows * cols].reshape(rows, cols)
+
+
+def _inputs(rows, cols, scale):
+    rng = np.random.default_rng(rows * 7919 + cols)
+    x = (rng.standard_normal((rows, cols)) * scale + 0.25).astype(np.float32)
+    return x, rng.uniform(0.5, 1.5, cols).astype(np.float32), rng.uniform(-0.5, 0.5, cols).astype(np.float32)
+
+
+def _close(op, got, want):
+    assert np.all(np.abs(got - want) <= 1e-5 * (1 + np.abs(want))), float(np.max(np.abs(got - want)))
+    if op == "softmax":
+        assert np.all(np.abs(got - want) <= 1e-5 * want + 1e-37)
+
+
+@pytest.mark.parametrize("op", OPS)
+@pytest.mark.parametrize("rows,cols", [
+    (3, 4), (5, 5), (2, 7), (9, 65), (4, 254), (3, 257), (5, 511), (3, 1001), (2, 2050), (3, 4099), (2, 8191),
+    (2, 16383), (2, 32767),                                     # ragged register plans, their last packs
+    (2, 32769), (3, 32772), (1, 36861), (2, 128256), (1, 131071), (33, 40002),   # 9 and 10 chunks and up
+    (1, (1 << 20) + 1), (1, 2_000_003)])                        # the 16-pack chunks
+@pytest.mark.parametrize("shift", [0, 1])
+def test_long_and_ragged_rows(ow, op, rows, cols, shift):
+    x, g, b = _inputs(rows, cols, 4.0 if op == "softmax" else 1.0)
+    _close(op, _run(ow, op, x, g, b, shift), _want(op, x, g, b))
+
+
+@pytest.mark.parametrize("op", OPS)
+@pytest.mark.parametrize("rows,cols", [(3, 5), (7, 1001), (2, 8191), (2, 40001)])
+def test_in_place(ow, op, rows, cols):
+    """In place, a long row cannot pass its statistics through the output and keeps one workgroup."""
+    x, g, b = _inputs(rows, cols, 2.0)
+    _close(op, _run(ow, op, x, g, b, 0, True), _want(op, x, g, b))
+
+
+@pytest.mark.parametrize("cols", [1001, 50003])
+def test_softmax_special_values(ow, cols):
+    """-inf entries (whole chunks of them) weigh nothing; a row of nothing but -inf, one with +inf and one
+    with a NaN are NaN throughout, and no row touches another."""
+    x, g, b = _inputs(5, cols, 1.0)
+    x[0, : cols - 3] = -np.inf
+    x[1, :] = -np.inf
+    x[2, 17] = np.inf
+    x[3, cols - 1] = np.nan
+    got = _run(ow, "softmax", x, g, b)
+    assert np.all(got[0, : cols - 3] == 0) and np.all(np.isnan(got[1:4]))
+    keep = [0, 4]
+    _close("softmax", got[keep], _want("softmax", x[keep], g, b))
