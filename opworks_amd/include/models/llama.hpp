@@ -728,8 +728,8 @@ template <typename WT> class LlamaModelT final : public LlamaRuntime {
     // bf16 on load from 16 rows (the reference's linear_mma_bf16 path,
     // models/llama.cuh:190-199), and below 16 rows the fp32 MFMA GEMM with fp32
     // inputs against the widened bf16 weights, as the reference's linear_dispatch does.
-    // Up to 64 rows every form runs on gemm_rows_kernel, which splits K inside its workgroups.
-    // Above, outputs with too few tiles to fill the GPU (o_proj, down, qkv at a few
+    // Short prompts run on gemm_rows_kernel, which splits K inside its workgroups (gemm_plan.hpp's
+    // costs say from where). Outputs with too few tiles to fill the GPU (o_proj, down, qkv at a few
     // hundred rows) split K across workgroups into the session's workspace.
     // `reduce` (optional, split-K outputs): run in place of the split-K reduction kernel, see
     // gemm_f32_launch_splitk. Returns true when K was split (and `reduce`, if given, ran).
@@ -780,7 +780,7 @@ template <typename WT> class LlamaModelT final : public LlamaRuntime {
                 reduce);
         } else { // the gate/up projection (SwiGLU store) on bf16x6 products, the others fp32 MFMA
             detail::gemm_f32_launch<detail::BLayout::nk, IdentityEpilogue, kStore>(
-                A, W, nullptr, C, M, N, K, IdentityEpilogue{}, st, 1, kStore == detail::GemmStore::swiglu);
+                A, W, nullptr, C, M, N, K, IdentityEpilogue{}, st, kStore == detail::GemmStore::swiglu);
         }
         return false;
     }

@@ -53,6 +53,10 @@ constexpr int kBfBM = 256, kBfBN = 256;
 constexpr int kBfBK = 32; // K granularity of split-K planning (the smaller of the two K tiles)
 constexpr int kBfThreads = 512;
 
+// Products of so few rows take gemm_rows_kernel.
+constexpr int kRowsMax = 64;
+inline bool gemm_rows_use(int M, int K) { return M <= kRowsMax && K > 0; }
+
 // Workgroup tile shapes. Big: 256 x 256 outputs, 8 waves in 2 x 4 (128 x 64 each), one
 // workgroup per CU. Small: 128 x 128, 4 waves in 2 x 2 (64 x 64 each), 64 KB of LDS so two
 // workgroups share a CU; for short-M products (prefill projections at a few hundred rows), where
@@ -534,7 +538,9 @@ void gemm_bf16_launch(const TA *A, const uint16_t *W, const float *bias, float *
             "swiglu epilogue needs an even number of columns");
     if constexpr (kStore != GemmStore::partial) {
         if (splits == 1 && gemm_rows_use(M, K)) {
-            gemm_rows_launch<std::is_same_v<TA, float>, Epi, kStore>(A, W, bias, C, M, N, K, epi, stream);
+            constexpr bool kRound = std::is_same_v<TA, float>;
+            const GemmPick pick = gemm_pick(kGemmCostWbf16, M, N, K, false, gemm_rows_staged_ok<BLayout::nk>(A, W, N, K));
+            gemm_tile_launch<BLayout::nk, kRound, Epi, kStore>(pick.tile, A, W, bias, C, M, N, K, epi, stream);
             return;
         }
     }

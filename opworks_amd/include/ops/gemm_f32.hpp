@@ -487,19 +487,11 @@ void gemm_f32_launch_shape(const float *A, const TB *B, const float *bias, float
 
 } // namespace opworks::detail
 
-#include "gemm_rows.hpp"
-#include "gemm_x6.hpp"
+#include "gemm_plan.hpp"
 
 namespace opworks::detail {
 
-// The fp32 products that the bf16x6 kernel takes: fp32 operands, A row-major, 16-byte aligned,
-// K a multiple of 8 (and N of 4 for a kn-layout B), and enough work to fill its 128 x 256 tiles
-// (at 4096^3 nk: 1003 -> 673 us, 1.30 of the fp32 MFMA peak; 512 x 16384 x 2048: 279 -> 179 us), for plain
-// and SwiGLU stores. Callers that need the fp32 MFMA kernels' summation pass allow_x6 = false; the
-// split-K form never takes it. The Llama runtime, held to the oracle's logits at NRMSE 1e-5, takes
-// it for the gate/up projection only: config 5's worst step read 9.27e-6 on fp32 MFMAs, 9.94e-6 with
-// gate/up on bf16x6 (fp32 TTFT 9.57 -> 8.10 ms), 1.05e-5 with every projection on it.
-// OPWORKS_GEMM_X6=0 in the environment keeps every product on the fp32 MFMA kernels.
+// OPWORKS_GEMM_X6=0 in the environment keeps every fp32 product on fp32 MFMAs.
 inline bool gemm_x6_enabled() {
     static const bool enabled = [] {
         const char *v = std::getenv("OPWORKS_GEMM_X6");
@@ -507,48 +499,63 @@ inline bool gemm_x6_enabled() {
     }();
     return enabled;
 }
-template <BLayout kB, GemmStore kStore, typename TB, ALayout kAL>
-inline bool gemm_use_x6(const float *A, const TB *B, int M, int N, int K) {
-    if constexpr (std::is_same_v<TB, float> && kAL == ALayout::mk &&
-                  (kStore == GemmStore::store || kStore == GemmStore::swiglu)) {
-        return M >= 16 && int64_t(M) * N * K >= (int64_t(1) << 26) && gemm_x6_ok<kB>(A, B, N, K) &&
-               gemm_x6_enabled();
-    } else {
-        return false;
-    }
+
+// The fp32-MFMA tile of a product when K is not split: GemmBig when its tiles alone cover every CU, else
+// GemmMid when its 256 x 128 tiles do (the prefill gate/up projection at 512 rows: 280 -> 262 us
+// against GemmSmall), else GemmSmall. Its cost in gemm_plan.hpp's model.
+inline GemmTileCost gemm_f32_tile_cost(int M, int N) {
+    if (blocks_for64(M, GemmBig::BM) * blocks_for64(N, GemmBig::BN) >= 256)
+        return {GemmTile::fp32_mfma, GemmBig::BM, GemmBig::BN, 3.f, 6.f, 7.6f};
+    if (blocks_for64(M, GemmMid::BM) * blocks_for64(N, GemmMid::BN) >= 256)
+        return {GemmTile::fp32_mfma, GemmMid::BM, GemmMid::BN, 3.f, 6.f, 4.f};
+    return {GemmTile::fp32_mfma, GemmSmall::BM, GemmSmall::BN, 2.9f, 5.8f, 2.9f};
 }
 
-// Enqueues C[M][N] = epi(A[M][K] B + bias) (written per kStore). K == 0 writes epi(bias or 0).
-// Up to 64 rows of an nk-layout product take gemm_rows_kernel.
-// When K is not split: GemmBig when its tiles alone cover every CU, else GemmMid when its
-// 256 x 128 tiles do (the prefill gate/up projection at 512 rows: 280 -> 262 us against
-// GemmSmall); otherwise, and for split-K partials, GemmSmall.
+// The kernel for an fp32-accuracy product with a row-major A (fp32 or, nk, bf16 weights). Callers that
+// need fp32 MFMAs' summation pass allow_parts = false: the Llama runtime, held to the oracle's logits
+// at NRMSE 1e-5, takes split operands for the gate/up projection only (config 5's worst step read
+// 9.27e-6 on fp32 MFMAs, 9.94e-6 with gate/up on bf16x6, 1.05e-5 with every projection on it).
+template <BLayout kB, GemmStore kStore, typename TB>
+inline GemmPick gemm_f32_pick(const float *A, const TB *B, int M, int N, int K, bool allow_parts) {
+    const bool parts = allow_parts && (kStore == GemmStore::store || kStore == GemmStore::swiglu) &&
+                       gemm_x6_ok<kB>(N, K) && gemm_x6_enabled();
+    const bool staged = gemm_rows_staged_ok<kB>(A, B, N, K);
+    GemmPick pick;
+    if constexpr (std::is_same_v<TB, float>)
+        pick = gemm_pick(kGemmCostF32, M, N, K, parts, staged);
+    else
+        pick = gemm_pick(kGemmCostWbf16, M, N, K, parts, staged);
+    if (!parts) { // with split operands allowed, one of their tiles is always cheaper
+        const float cost = gemm_cost(gemm_f32_tile_cost(M, N), M, N, K, cu_count());
+        if (cost < pick.cost)
+            pick = {GemmTile::fp32_mfma, cost};
+    }
+    return pick;
+}
+
+// Enqueues C[M][N] = epi(A[M][K] B + bias) (written per kStore). K == 0 writes epi(bias or 0). The
+// kernel is gemm_f32_pick's, or the fp32-MFMA tiles for a column-major A.
 template <BLayout kB, typename Epi, GemmStore kStore = GemmStore::store, typename TB = float,
           ALayout kAL = ALayout::mk>
 void gemm_f32_launch(const float *A, const TB *B, const float *bias, float *C, int M, int N, int K, Epi epi,
-                     hipStream_t stream, int splits = 1, bool allow_x6 = true) {
+                     hipStream_t stream, bool allow_parts = true) {
     require(kStore != GemmStore::swiglu || N % 2 == 0, "swiglu epilogue needs an even number of columns");
-    if constexpr (kB == BLayout::nk && kAL == ALayout::mk && kStore != GemmStore::partial) {
-        if (splits == 1 && gemm_rows_use(M, K)) {
-            gemm_rows_launch<false, Epi, kStore>(A, B, bias, C, M, N, K, epi, stream);
-            return;
+    if constexpr (kAL == ALayout::mk) {
+        if (K > 0) {
+            const GemmPick pick = gemm_f32_pick<kB, kStore, TB>(A, B, M, N, K, allow_parts);
+            if (pick.tile != GemmTile::fp32_mfma) {
+                gemm_tile_launch<kB, false, Epi, kStore>(pick.tile, A, B, bias, C, M, N, K, epi, stream);
+                return;
+            }
         }
     }
-    if constexpr (std::is_same_v<TB, float> && kAL == ALayout::mk &&
-                  (kStore == GemmStore::store || kStore == GemmStore::swiglu)) {
-        if (allow_x6 && gemm_use_x6<kB, kStore, TB, kAL>(A, B, M, N, K)) {
-            gemm_x6_launch<kB, Epi, kStore>(A, B, bias, C, M, N, K, epi, stream, splits);
-            return;
-        }
-    }
-    const int64_t big_tiles = blocks_for64(M, GemmBig::BM) * blocks_for64(N, GemmBig::BN);
-    const int64_t mid_tiles = blocks_for64(M, GemmMid::BM) * blocks_for64(N, GemmMid::BN);
-    if (splits == 1 && big_tiles >= 256)
-        gemm_f32_launch_shape<GemmBig, kB, Epi, kStore, TB, kAL>(A, B, bias, C, M, N, K, epi, stream, splits);
-    else if (splits == 1 && mid_tiles >= 256)
-        gemm_f32_launch_shape<GemmMid, kB, Epi, kStore, TB, kAL>(A, B, bias, C, M, N, K, epi, stream, splits);
+    const GemmTileCost tile = gemm_f32_tile_cost(M, N);
+    if (tile.bm == GemmBig::BM && tile.bn == GemmBig::BN)
+        gemm_f32_launch_shape<GemmBig, kB, Epi, kStore, TB, kAL>(A, B, bias, C, M, N, K, epi, stream, 1);
+    else if (tile.bm == GemmMid::BM)
+        gemm_f32_launch_shape<GemmMid, kB, Epi, kStore, TB, kAL>(A, B, bias, C, M, N, K, epi, stream, 1);
     else
-        gemm_f32_launch_shape<GemmSmall, kB, Epi, kStore, TB, kAL>(A, B, bias, C, M, N, K, epi, stream, splits);
+        gemm_f32_launch_shape<GemmSmall, kB, Epi, kStore, TB, kAL>(A, B, bias, C, M, N, K, epi, stream, 1);
 }
 
 // Floats of split-K workspace any launch planned by splitk_factor(tiles, ., 512) needs.
@@ -566,10 +573,6 @@ bool gemm_f32_launch_splitk(const float *A, const TB *B, const float *bias, floa
     // K at all, else on GemmSmall tiles up to 512 (prefill at 512 rows: qkv 86.2 -> 81.8 us, down
     // 152.5 -> 148.4 us, o_proj unchanged). Either plan needs at most 256 * 256 * 128 =
     // 512 * 128 * 128 floats.
-    if (kB == BLayout::nk && gemm_rows_use(M, K)) { // splits K inside its workgroups
-        gemm_f32_launch<kB, Epi, kStore, TB>(A, B, bias, C, M, N, K, epi, stream, 1, false);
-        return false;
-    }
     const int ktiles = static_cast<int>(blocks_for64(K, kGemmBK));
     const int mid_splits =
         M >= GemmMid::BM
@@ -579,9 +582,20 @@ bool gemm_f32_launch_splitk(const float *A, const TB *B, const float *bias, floa
                                       : splitk_factor(static_cast<int>(blocks_for64(M, GemmSmall::BM) *
                                                                        blocks_for64(N, GemmSmall::BN)),
                                                       ktiles, 512);
+    // The same product without a split, when that is no dearer: the few-row tiles split K inside
+    // their workgroups, and the partial tiles' sum is a launch and a pass of its own (down at 128
+    // rows: 91 us with it, 48 without). Up to 256 rows: above, the two are within 15% of each other,
+    // and the 512-token prefill's logits, held to the oracle at NRMSE 1e-5, read 9.94e-6 with the
+    // split sums and 1.01e-5 with the few-row tiles'.
+    const int splits_bm = mid_splits > 1 ? GemmMid::BM : GemmSmall::BM;
+    const float tile_c = mid_splits > 1 ? 4.f : 2.9f;
+    const int64_t split_tiles = blocks_for64(M, splits_bm) * blocks_for64(N, GemmSmall::BN) * splits;
+    const float split_cost = 8.f + static_cast<float>(blocks_for64(split_tiles, cu_count())) *
+                                       (6.f + tile_c * static_cast<float>(K) / (32.f * static_cast<float>(splits)));
     if (splits == 1 || N % 4 != 0 || !ws || int64_t(splits) * M * N > ws_floats || !aligned16(C) ||
-        (bias && !aligned16(bias))) {
-        gemm_f32_launch<kB, Epi, kStore, TB>(A, B, bias, C, M, N, K, epi, stream, 1, false); // fp32 MFMA
+        (bias && !aligned16(bias)) ||
+        (M <= 256 && gemm_f32_pick<kB, kStore, TB>(A, B, M, N, K, false).cost <= split_cost)) {
+        gemm_f32_launch<kB, Epi, kStore, TB>(A, B, bias, C, M, N, K, epi, stream, false); // fp32 MFMA
         return false;
     }
     if (mid_splits > 1)

@@ -1,0 +1,136 @@
+#pragma once
+
+// Which GEMM kernel and tile takes a product: the cheapest by a measured cost model.
+//
+// A kernel's time on an MI355X is close to
+//     t0 + rounds * (a + c * K / 32) microseconds,   rounds = ceil(tiles / CUs):
+// a launch, and per round of tiles a start and end (a) and the K steps (c per 32 k, which holds the
+// step's chain of loads, LDS accesses, splits and MFMAs on one CU). t0, a and c below are least-squares
+// fits to HIP-event times of about 100 products per form, M 9..4096, N 64..16384, K 64..8192, odd sizes
+// among them, each product on every tile (rms error 5-15%). On those products the tile the model
+// picks costs 0.4-1.2% (fp32) and 2% (bf16 weights) more than the fastest one, in the geometric mean.
+//
+// Small tiles finish few outputs per step but spread a small product over the whole chip; large ones
+// re-read their operands least. E.g. fp32 1000 x 1001, K = 1500: 34-39 us on 64 x 64 tiles (256 of
+// them), 48 on 64 x 128, 64-71 on 128 x 128, 106-111 on 128 x 256, 123-180 on the 128 x 128 fp32-MFMA
+// tiles; 128 x 8192, K = 2048: 42, 53, 80, 133 and 163; 4096^3: 128 x 256 fastest.
+
+// Included by gemm_f32.hpp after the kernels it chooses from.
+
+#include <cstdint>
+
+#include "../core/hip_utils.hpp"
+#include "gemm_rows.hpp"
+#include "gemm_x6.hpp"
+
+namespace opworks::detail {
+
+enum class GemmTile {
+    parts128x256, // gemm_x6_kernel, any alignment
+    parts128x128,
+    parts64x128,
+    parts64x64,
+    staged16x16, // gemm_rows_kernel through LDS, rows on the 16-byte grid
+    staged32x32,
+    staged64x32,
+    direct16x16, // gemm_rows_kernel straight from memory, any alignment
+    direct32x32,
+    fp32_mfma, // gemm_f32_mfma_kernel
+};
+
+struct GemmTileCost {
+    GemmTile tile;
+    int bm, bn;
+    float t0, a, c;
+};
+struct GemmPick {
+    GemmTile tile;
+    float cost;
+};
+
+inline float gemm_cost(const GemmTileCost &t, int M, int N, int K, int cus) {
+    const int64_t tiles = blocks_for64(M, t.bm) * blocks_for64(N, t.bn);
+    return t.t0 + static_cast<float>(blocks_for64(tiles, cus)) * (t.a + t.c * static_cast<float>(K) / 32.f);
+}
+
+// fp32 x fp32, both B layouts
+inline constexpr GemmTileCost kGemmCostF32[] = {
+    {GemmTile::parts128x256, 128, 256, 6.f, 5.4f, 2.0f}, {GemmTile::parts128x128, 128, 128, 0.f, 6.6f, 1.28f},
+    {GemmTile::parts64x128, 64, 128, 0.6f, 6.5f, 0.8f},  {GemmTile::parts64x64, 64, 64, 0.5f, 4.4f, 0.58f},
+    {GemmTile::staged16x16, 16, 16, 2.f, 0.53f, 0.072f}, {GemmTile::staged32x32, 32, 32, 1.f, 2.f, 0.175f},
+    {GemmTile::staged64x32, 64, 32, 0.65f, 3.1f, 0.305f}, {GemmTile::direct16x16, 16, 16, 2.f, 0.3f, 0.1f},
+    {GemmTile::direct32x32, 32, 32, 1.5f, 1.2f, 0.23f},
+};
+// fp32 X, bf16 W
+inline constexpr GemmTileCost kGemmCostWbf16[] = {
+    {GemmTile::parts128x256, 128, 256, 0.f, 8.6f, 1.08f}, {GemmTile::parts64x128, 64, 128, 6.3f, 0.f, 0.466f},
+    {GemmTile::parts64x64, 64, 64, 4.4f, 0.f, 0.37f},     {GemmTile::staged16x16, 16, 16, 1.5f, 1.4f, 0.05f},
+    {GemmTile::staged32x32, 32, 32, 1.6f, 2.2f, 0.18f},   {GemmTile::staged64x32, 64, 32, 1.35f, 3.6f, 0.305f},
+    {GemmTile::direct16x16, 16, 16, 2.5f, 0.f, 0.091f},   {GemmTile::direct32x32, 32, 32, 4.5f, 0.f, 0.19f},
+};
+
+inline bool gemm_tile_is_parts(GemmTile t) {
+    return t == GemmTile::parts128x256 || t == GemmTile::parts128x128 || t == GemmTile::parts64x128 ||
+           t == GemmTile::parts64x64;
+}
+inline bool gemm_tile_is_staged(GemmTile t) {
+    return t == GemmTile::staged16x16 || t == GemmTile::staged32x32 || t == GemmTile::staged64x32;
+}
+
+// The cheapest tile of `table`: the split-operand ones only with `parts`, the staged ones only with
+// `staged`, the direct ones only without.
+template <size_t n>
+inline GemmPick gemm_pick(const GemmTileCost (&table)[n], int M, int N, int K, bool parts, bool staged) {
+    const int cus = cu_count();
+    GemmPick best{GemmTile::fp32_mfma, 3.4e38f};
+    for (const GemmTileCost &t : table) {
+        const bool usable = gemm_tile_is_parts(t.tile) ? parts : gemm_tile_is_staged(t.tile) ? staged : !staged;
+        if (!usable)
+            continue;
+        const float cost = gemm_cost(t, M, N, K, cus);
+        if (cost < best.cost)
+            best = {t.tile, cost};
+    }
+    return best;
+}
+
+// The tiles' kernel shapes.
+using GemmParts128x256 = GemmX6Shape<128, 256, 2, 4, 1>;
+using GemmParts128x128 = GemmX6Shape<128, 128, 2, 4, 1>;
+using GemmParts64x128 = GemmX6Shape<64, 128, 2, 2, 2>;
+using GemmParts64x64 = GemmX6Shape<64, 64, 2, 2, 2>;
+using GemmRows16x16 = RowsShape<1, 1, 8, 2>;
+using GemmRows32x32 = RowsShape<2, 2, 4, 3>;
+using GemmRows64x32 = RowsShape<4, 2, 4, 2>;
+
+template <BLayout kB, bool kRound, typename Epi, GemmStore kStore, typename TA, typename TB>
+void gemm_tile_launch(GemmTile tile, const TA *A, const TB *B, const float *bias, float *C, int M, int N, int K,
+                      Epi epi, hipStream_t stream) {
+    auto rows = [&](auto shape, auto staged) {
+        gemm_rows_launch<decltype(shape), kB, kRound, decltype(staged)::value, Epi, kStore>(A, B, bias, C, M, N, K,
+                                                                                           epi, stream);
+    };
+    auto parts = [&](auto shape) {
+        if constexpr (kStore == GemmStore::store || kStore == GemmStore::swiglu)
+            gemm_x6_launch<decltype(shape), kB, kRound, Epi, kStore>(A, B, bias, C, M, N, K, epi, stream);
+        else
+            throw std::invalid_argument("gemm: no split-operand kernel for this store");
+    };
+    switch (tile) {
+    case GemmTile::parts128x256: parts(GemmParts128x256{}); break;
+    case GemmTile::parts128x128:
+        if constexpr (std::is_same_v<TB, float>)
+            parts(GemmParts128x128{});
+        break;
+    case GemmTile::parts64x128: parts(GemmParts64x128{}); break;
+    case GemmTile::parts64x64: parts(GemmParts64x64{}); break;
+    case GemmTile::staged16x16: rows(GemmRows16x16{}, std::true_type{}); break;
+    case GemmTile::staged32x32: rows(GemmRows32x32{}, std::true_type{}); break;
+    case GemmTile::staged64x32: rows(GemmRows64x32{}, std::true_type{}); break;
+    case GemmTile::direct16x16: rows(GemmRows16x16{}, std::false_type{}); break;
+    case GemmTile::direct32x32: rows(GemmRows32x32{}, std::false_type{}); break;
+    case GemmTile::fp32_mfma: throw std::invalid_argument("gemm: the fp32-MFMA tiles have their own launcher");
+    }
+}
+
+} // namespace opworks::detail

@@ -82,12 +82,29 @@ __device__ __forceinline__ bf16x8v raw8_bf16(const Raw8<float> &r) {
 }
 __device__ __forceinline__ bf16x8v raw8_bf16(const Raw8<uint16_t> &r) { return __builtin_bit_cast(bf16x8v, r.v); }
 
+__device__ __forceinline__ void raw8_split(const Raw8<float> &r, bf16x8v (&part)[3]) {
+    const float x[8] = {r.v[0][0], r.v[0][1], r.v[0][2], r.v[0][3], r.v[1][0], r.v[1][1], r.v[1][2], r.v[1][3]};
+    split3x8(x, part);
+}
+__device__ __forceinline__ void raw8_mask(Raw8<float> &r, bool keep) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+        r.v[j / 4][j % 4] = keep ? r.v[j / 4][j % 4] : 0.f;
+}
+__device__ __forceinline__ void raw8_mask(Raw8<uint16_t> &r, bool keep) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        r.v[j] = keep ? r.v[j] : 0u;
+}
+__device__ __forceinline__ float as_float(float x) { return x; }
+__device__ __forceinline__ float as_float(uint16_t bits) { return __uint_as_float(uint32_t(bits) << 16); }
+
 // Tile shape: 16 FM rows x 16 FN columns per workgroup, kWaves waves over K, kDepth steps in flight.
 template <int kFM, int kFN, int kW, int kD> struct RowsShape {
     static constexpr int FM = kFM, FN = kFN, kWaves = kW, kDepth = kD, kThreads = kW * kWaveSize;
 };
 
-template <typename S, typename TX, typename TW, bool kRound, bool kStaged, typename Epi, GemmStore kStore>
+template <typename S, BLayout kB, typename TX, typename TW, bool kRound, bool kStaged, typename Epi, GemmStore kStore>
 __global__ __launch_bounds__(S::kThreads) void gemm_rows_kernel(const TX *__restrict__ X, const TW *__restrict__ W,
                                                                 const float *__restrict__ bias, float *__restrict__ C,
                                                                 int M, int N, int K, Epi epi) {
@@ -95,6 +112,7 @@ __global__ __launch_bounds__(S::kThreads) void gemm_rows_kernel(const TX *__rest
     constexpr bool kF32X = std::is_same_v<TX, float>, kF32W = std::is_same_v<TW, float>;
     static_assert(!kF32W || (kF32X && !kRound), "fp32 weights take fp32 inputs");
     constexpr bool kF32Mfma = kF32X && !kRound;
+    static_assert(kB == BLayout::nk || kF32W, "a kn-layout W is fp32");
     constexpr int kU = kF32W ? 1 : 2, kStep = 32 * kU; // K step: 128 bytes of each weight row
     // Staged steps: blocks of 16 rows x 128 bytes, FN of W, then FM x kXB of X.
     constexpr int kXB = kF32X && !kF32W ? 2 : 1, kXHalf = 128 / int(sizeof(TX)); // X elements per block row
@@ -105,7 +123,12 @@ __global__ __launch_bounds__(S::kThreads) void gemm_rows_kernel(const TX *__rest
     const int lane = threadIdx.x % kWaveSize;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
     const int l16 = lane % 16, quad = lane / 16;
-    const int n0 = blockIdx.x * 16 * FN, m0 = blockIdx.y * 16 * FM;
+    // Groups of 8 column tiles, row tile by row tile: a column tile's workgroups are 8 apart, so they
+    // run on one XCD (dispatch is round-robin) and share its weights through that L2.
+    const int tiles_m = (M + 16 * FM - 1) / (16 * FM), tiles_n = (N + 16 * FN - 1) / (16 * FN);
+    const int group = static_cast<int>(blockIdx.x / (8u * tiles_m)), in_group = blockIdx.x - group * 8 * tiles_m;
+    const int width = tiles_n - 8 * group < 8 ? tiles_n - 8 * group : 8;
+    const int n0 = (8 * group + in_group % width) * 16 * FN, m0 = in_group / width * 16 * FM;
     if (kStaged && M < 0) // never: an ordinary store, so the compiler keeps the reads of the direct loads
         lds[threadIdx.x] = 0;
 
@@ -120,6 +143,10 @@ __global__ __launch_bounds__(S::kThreads) void gemm_rows_kernel(const TX *__rest
     // Staged loads: instruction h of a block covers its rows 8 h .. 8 h + 7, lane l row 8 h + l / 8,
     // 16-byte slot l % 8, which holds chunk (l % 8) ^ ((row >> 1) & 7) of that row's 128 bytes.
     const int s_row = lane >> 3;
+    // A kn-layout W: rows of 16 FN columns, k = 8 q + e of the step in LDS row 4 e + q, so that the four
+    // quads' rows of one MFMA step lie side by side; with 128-byte rows the halves of rows q = 2, 3 are
+    // swapped, which puts the four 64-byte pieces on different banks.
+    constexpr int kLanesKn = 4 * FN, kRowsKn = kWaveSize / kLanesKn; // lanes per row, rows per instruction
     const TW *wsrc[FN][2];
     const TX *xsrc[FM][2];
     if constexpr (kStaged) {
@@ -127,8 +154,16 @@ __global__ __launch_bounds__(S::kThreads) void gemm_rows_kernel(const TX *__rest
         for (int h = 0; h < 2; ++h) {
             const int r = 8 * h + s_row, chunk = (lane & 7) ^ ((r >> 1) & 7);
 #pragma unroll
-            for (int j = 0; j < FN; ++j)
-                wsrc[j][h] = w_row(16 * j + r) + chunk * (16 / int(sizeof(TW)));
+            for (int j = 0; j < FN; ++j) {
+                if constexpr (kB == BLayout::nk) {
+                    wsrc[j][h] = w_row(16 * j + r) + chunk * (16 / int(sizeof(TW)));
+                } else {
+                    static_assert(FN <= 2, "the kn swizzle covers rows of 64 or 128 bytes");
+                    const int p = (2 * j + h) * kRowsKn + lane / kLanesKn, q = p & 3;
+                    const int col = n0 + 4 * ((lane % kLanesKn) ^ (FN == 2 ? 4 * (q >> 1) : 0));
+                    wsrc[j][h] = W + int64_t(8 * q + p / 4) * N + (col < N ? col : N - 4); // N % 4 == 0
+                }
+            }
 #pragma unroll
             for (int i = 0; i < FM; ++i)
                 xsrc[i][h] = x_row(16 * i + r) + chunk * (16 / int(sizeof(TX)));
@@ -142,7 +177,8 @@ __global__ __launch_bounds__(S::kThreads) void gemm_rows_kernel(const TX *__rest
         for (int j = 0; j < FN; ++j)
 #pragma unroll
             for (int h = 0; h < 2; ++h)
-                load_lds16(wsrc[j][h] + k, reinterpret_cast<uint16_t *>(st + j * 2048 + h * 1024));
+                load_lds16(wsrc[j][h] + (kB == BLayout::nk ? int64_t(k) : int64_t(k) * N),
+                           reinterpret_cast<uint16_t *>(st + j * 2048 + h * 1024));
 #pragma unroll
         for (int i = 0; i < FM; ++i)
 #pragma unroll
@@ -169,8 +205,17 @@ __global__ __launch_bounds__(S::kThreads) void gemm_rows_kernel(const TX *__rest
 #pragma unroll
         for (int u = 0; u < kU; ++u) {
 #pragma unroll
-            for (int j = 0; j < FN; ++j)
-                get(f.w[j][u], st + j * 2048, u);
+            for (int j = 0; j < FN; ++j) {
+                if constexpr (kB == BLayout::nk) {
+                    get(f.w[j][u], st + j * 2048, u);
+                } else {
+                    const int half = FN == 2 ? 64 * (j ^ (quad >> 1)) : 0;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        f.w[j][u].v[e / 4][e % 4] =
+                            *reinterpret_cast<const float *>(st + (4 * e + quad) * (64 * FN) + half + 4 * l16);
+                }
+            }
 #pragma unroll
             for (int i = 0; i < FM; ++i)
                 get(f.x[i][u], st + (FN + i * kXB) * 2048, u);
@@ -181,8 +226,16 @@ __global__ __launch_bounds__(S::kThreads) void gemm_rows_kernel(const TX *__rest
         for (int u = 0; u < kU; ++u) {
             const int k = step * kStep + 32 * u + 8 * quad;
 #pragma unroll
-            for (int j = 0; j < FN; ++j)
-                raw8_load(f.w[j][u], w_row(16 * j + l16) + k);
+            for (int j = 0; j < FN; ++j) {
+                if constexpr (kB == BLayout::nk) {
+                    raw8_load(f.w[j][u], w_row(16 * j + l16) + k);
+                } else {
+                    const int n = n0 + 16 * j + l16;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        f.w[j][u].v[e / 4][e % 4] = W[int64_t(k + e) * N + (n < N ? n : N - 1)];
+                }
+            }
 #pragma unroll
             for (int i = 0; i < FM; ++i)
                 raw8_load(f.x[i][u], x_row(16 * i + l16) + k);
@@ -194,8 +247,18 @@ __global__ __launch_bounds__(S::kThreads) void gemm_rows_kernel(const TX *__rest
             const int k = step * kStep + 32 * u + 8 * quad;
             const int at = k < K ? k : K - 1;
 #pragma unroll
-            for (int j = 0; j < FN; ++j)
-                raw8_load_tail(f.w[j][u], w_row(16 * j + l16) + at, K - k);
+            for (int j = 0; j < FN; ++j) {
+                if constexpr (kB == BLayout::nk) {
+                    raw8_load_tail(f.w[j][u], w_row(16 * j + l16) + at, K - k);
+                } else {
+                    const int n = n0 + 16 * j + l16;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        const float v = W[int64_t(k + e < K ? k + e : K - 1) * N + (n < N ? n : N - 1)];
+                        f.w[j][u].v[e / 4][e % 4] = k + e < K ? v : 0.f;
+                    }
+                }
+            }
 #pragma unroll
             for (int i = 0; i < FM; ++i)
                 raw8_load_tail(f.x[i][u], x_row(16 * i + l16) + at, K - k);
@@ -361,42 +424,24 @@ __global__ __launch_bounds__(S::kThreads) void gemm_rows_kernel(const TX *__rest
     }
 }
 
-// Whether few-row products take this kernel: the tiled kernels' M padding costs more than its extra
-// reads of X up to 64 rows (N = 8192, K = 2048, fp32: 25 us against 157; at 100 rows 47).
-constexpr int kRowsMax = 64;
-inline bool gemm_rows_use(int M, int K) { return M <= kRowsMax && K > 0; }
+// Whether a product's rows lie on the 16-byte grid that the staged form reads (kn: W's rows of N).
+template <BLayout kB, typename TX, typename TW> inline bool gemm_rows_staged_ok(const TX *X, const TW *W, int N, int K) {
+    constexpr int kAlign = 16 / (sizeof(TX) < sizeof(TW) ? sizeof(TX) : sizeof(TW));
+    return aligned16(X) && aligned16(W) && K % kAlign == 0 && (kB == BLayout::nk || (N % 4 == 0 && N >= 4));
+}
 
-// C (per kStore) = epi(X[M][K] W[N][K]^T + bias). The largest tile that fits the rows and still gives
-// every CU a workgroup: it reads X from L2 the fewest times; below that, 16 x 16 tiles, for the most
-// workgroups. (fp32 weights, M <= 16, 8192 columns: 16 x 16 tiles 14.4 us on 512 workgroups, 16 x 32
-// 18.5 on 256, so there only bf16 weights, half the bytes per tile, take the wide tile: 11.4 against
-// 13.8.)
-template <bool kRound, typename Epi, GemmStore kStore, typename TX, typename TW>
+template <typename S, BLayout kB, bool kRound, bool kStaged, typename Epi, GemmStore kStore, typename TX, typename TW>
 void gemm_rows_launch(const TX *X, const TW *W, const float *bias, float *C, int M, int N, int K, Epi epi,
                       hipStream_t stream) {
-    auto run = [&](auto shape, auto staged) {
-        using S = decltype(shape);
-        const dim3 grid(static_cast<unsigned>(blocks_for64(N, 16 * S::FN)),
-                        static_cast<unsigned>(blocks_for64(M, 16 * S::FM)));
-        launch_async(stream, gemm_rows_kernel<S, TX, TW, kRound, decltype(staged)::value, Epi, kStore>, grid,
-                     S::kThreads, X, W, bias, C, M, N, K, epi);
-    };
-    using Small = RowsShape<1, 1, 8, 2>;
-    constexpr int kAlign = 16 / sizeof(TW); // elements of X are as wide as W's, or wider
-    if (!aligned16(X) || !aligned16(W) || K % kAlign != 0) {
-        run(Small{}, std::false_type{});
-        return;
-    }
-    const int cus = cu_count();
-    auto fills = [&](int fm, int fn) { return blocks_for64(M, 16 * fm) * blocks_for64(N, 16 * fn) >= cus; };
-    if (M > 32 && fills(4, 2))
-        run(RowsShape<4, 2, 4, 2>{}, std::true_type{});
-    else if (M > 16 && fills(2, 2))
-        run(RowsShape<2, 2, 4, 3>{}, std::true_type{});
-    else if ((M > 16 || !std::is_same_v<TW, float>) && fills(1, 2))
-        run(RowsShape<1, 2, 8, 2>{}, std::true_type{});
-    else
-        run(Small{}, std::true_type{});
+    require((kStore != GemmStore::swiglu && kStore != GemmStore::swiglu_bf16) || N % 2 == 0,
+            "swiglu epilogue needs an even number of columns");
+    require(M > 0 && N > 0 && K > 0, "gemm_rows: empty product");
+    if constexpr (kStaged)
+        require(gemm_rows_staged_ok<kB>(X, W, N, K), "gemm_rows: rows must lie on the 16-byte grid");
+    const int64_t tiles_m = blocks_for64(M, 16 * S::FM), tiles_n = blocks_for64(N, 16 * S::FN);
+    require(tiles_m * tiles_n <= INT32_MAX, "gemm_rows: grid too large");
+    launch_async(stream, gemm_rows_kernel<S, kB, TX, TW, kRound, kStaged, Epi, kStore>,
+                 static_cast<int>(tiles_m * tiles_n), S::kThreads, X, W, bias, C, M, N, K, epi);
 }
 
 } // namespace opworks::detail

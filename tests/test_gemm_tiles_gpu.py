@@ -1,0 +1,136 @@
+"""The fp32-accuracy GEMM on each tile that gemm_plan.hpp can pick, at sizes inside that tile's range whose
+edges are partial (rows, columns, K steps), for both B layouts, fp32 and bf16 weights, and operands off
+the 16-byte grid; and values that three bf16 parts cannot hold: infinities, NaNs, magnitudes near the
+largest and the smallest normal number.
+
+Tolerance: each product is within 2^-23 of its value (three-part operands; exact or once rounded
+otherwise), and a sum of K terms in fp32 in any order within (K + 1) 2^-23 of sum |a b|."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+# (M, out, inner), and the tile the cost model gives it
+ALIGNED = [
+    (1238, 5624, 584),   # 128 x 256
+    (951, 2280, 168),    # 128 x 128
+    (4090, 516, 512),    # 64 x 128
+    (522, 1440, 1512),   # 64 x 64
+    (232, 304, 2288),    # 16 x 16 staged
+    (195, 2296, 552),    # 32 x 32 staged
+    (754, 568, 1032),    # 64 x 32 staged
+]
+RAGGED = [
+    (1237, 5621, 583), (858, 2283, 169), (4087, 514, 509), (435, 1441, 1513),
+    (174, 305, 2289),    # 16 x 16 direct
+    (143, 2301, 559),    # 32 x 32 direct
+    (70, 67, 63), (129, 65, 9), (200, 3, 300), (90, 130, 5), (66, 4, 8), (130, 1, 1),
+    (435, 1440, 1512 + 4),   # inner a multiple of 4, not of 8
+    (435, 1442, 1512),       # the columns of a row-major B off the grid, its inner dimension on it
+]
+
+
+def _bf16(a):
+    u = np.ascontiguousarray(a, np.float32).view(np.uint32)
+    b = ((u.astype(np.uint64) + 0x7FFF + ((u >> 16) & 1)) >> 16).astype(np.uint16)
+    return b, (b.astype(np.uint32) << 16).view(np.float32)
+
+
+def _run(ow, a, w, form, act="none", bias=None, shift=0):
+    """form nk: w [out][inner]; kn: the same weights passed as [inner][out]; wbf16: nk in bf16 bits."""
+    m, k = a.shape
+    n = w.shape[0]
+
+    def up(x):
+        x = np.ascontiguousarray(x)
+        return ow.DeviceBuffer.from_host(np.concatenate([np.zeros(shift, x.dtype), x.reshape(-1)])).offset(shift)
+
+    da = up(a)
+    out = up(np.concatenate([np.full(m * n, 7, np.float32), np.full(8, 3, np.float32)]))
+    db = None if bias is None else up(bias)
+    if form == "wbf16":
+        dw = up(_bf16(w)[0])
+        ow.ops.linear_wbf16(da, dw, out, m, k, n)
+    else:
+        dw = up(w.T if form == "kn" else w)
+        ow.ops.mat_mul_fused(da, dw, db, out, m, k, n, form == "nk", act)
+    got = out.to_host()
+    assert np.array_equal(got[m * n:], np.full(8, 3, np.float32))
+    return got[:m * n].reshape(m, n)
+
+
+def _check(got, a, w, bias=None, act="none"):
+    a64, w64 = a.astype(np.float64), w.astype(np.float64)
+    b64 = 0.0 if bias is None else bias.astype(np.float64)
+    want = a64 @ w64.T + b64
+    bound = (a.shape[1] + 3) * 2.0 ** -23 * (np.abs(a64) @ np.abs(w64).T + np.abs(b64)) + 1e-37
+    if act == "relu":
+        want = np.maximum(want, 0)
+    worst = float(np.max(np.abs(got - want) / bound))
+    assert worst <= 1.0, worst
+
+
+def _data(m, n, k):
+    rng = np.random.default_rng(m * 31 + n * 7 + k)
+    return (rng.standard_normal((m, k), np.float32), rng.standard_normal((n, k), np.float32),
+            rng.uniform(-1, 1, n).astype(np.float32))
+
+
+@pytest.mark.parametrize("m,n,k", ALIGNED + RAGGED)
+@pytest.mark.parametrize("form", ["nk", "kn", "wbf16"])
+def test_tiles_match_float64(ow, m, n, k, form):
+    a, w, bias = _data(m, n, k)
+    if form == "wbf16":
+        w = _bf16(w)[1]
+        _check(_run(ow, a, w, form), a, w)
+    else:
+        _check(_run(ow, a, w, form, "relu", bias), a, w, bias, "relu")
+
+
+@pytest.mark.parametrize("m,n,k", [(951, 520, 168), (435, 1440, 520), (232, 304, 264), (100, 8, 40)])
+@pytest.mark.parametrize("form", ["nk", "kn", "wbf16"])
+@pytest.mark.parametrize("shift", [1, 2])
+def test_operands_off_the_grid(ow, m, n, k, form, shift):
+    a, w, bias = _data(m, n, k)
+    if form == "wbf16":
+        w = _bf16(w)[1]
+    _check(_run(ow, a, w, form, shift=shift), a, w)
+
+
+@pytest.mark.parametrize("m,n,k", [(951, 520, 168), (435, 1441, 169), (232, 304, 264), (129, 67, 65)])
+@pytest.mark.parametrize("form", ["nk", "kn", "wbf16"])
+def test_special_values(ow, m, n, k, form):
+    """Infinities and NaNs reach exactly the outputs that fp32 products give them; the largest finite value
+    (which rounds to infinity in bf16) keeps its finite products."""
+    rng = np.random.default_rng(k)
+    a = rng.uniform(0.5, 1.5, (m, k)).astype(np.float32)
+    w = _bf16(rng.uniform(0.5, 1.5, (n, k)).astype(np.float32))[1]
+    a[3, k - 1] = np.inf
+    a[5, 0] = np.nan
+    w[2, 1] = -np.inf
+    a[7, 2] = np.finfo(np.float32).max
+    w[:, 2] *= 2.0 ** -20
+    got = _run(ow, a, w, form)
+    with np.errstate(invalid="ignore"):
+        want = a.astype(np.float64) @ w.astype(np.float64).T
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(np.isposinf(got), np.isposinf(want)) and np.array_equal(np.isneginf(got), np.isneginf(want))
+    rows = [i for i in range(m) if i not in (3, 5)]
+    cols = [j for j in range(n) if j != 2]
+    _check(got[np.ix_(rows, cols)], a[rows], w[cols])
+
+
+@pytest.mark.parametrize("m,n,k", [(951, 520, 168), (232, 304, 264), (435, 1441, 169)])
+@pytest.mark.parametrize("form", ["nk", "kn", "wbf16"])
+@pytest.mark.parametrize("e", [-100, -120])
+def test_smallest_normal_inputs(ow, m, n, k, form, e):
+    """Inputs around 2^e, whose lower parts are subnormal in bf16, against weights that bring the products
+    back to 2^-10. Three bf16 parts hold a value to within 2^-134, half of bf16's subnormal spacing."""
+    a, w, _ = _data(m, n, k)
+    w = _bf16(w)[1]
+    a, w = a * np.float32(2.0 ** e), w * np.float32(2.0 ** (-e - 10))
+    got = _run(ow, a, w, form)
+    a64, w64 = a.astype(np.float64), w.astype(np.float64)
+    absw = np.abs(w64)
+    bound = (k + 3) * 2.0 ** -23 * (np.abs(a64) @ absw.T) + 2.0 ** -134 * absw.sum(1)[None, :]
+    assert float(np.max(np.abs(got - a64 @ w64.T) / bound)) <= 1.0
