@@ -808,7 +808,6 @@ template <typename WT> class LlamaModelT final : public LlamaRuntime {
                 A, reinterpret_cast<const uint16_t *>(W), nullptr, C, n, N, K, IdentityEpilogue{},
                 s.workspace.splitk.data(), s.workspace.splitk.size(), st);
         };
-        using StoreTag = std::integral_constant<GemmStore, GemmStore::store>;
         using ResidualTag = std::integral_constant<GemmStore, GemmStore::residual>;
         using SwigluBf16Tag = std::integral_constant<GemmStore, GemmStore::swiglu_bf16>;
         float *hidden = s.workspace.hidden.data(), *normed = s.workspace.normed.data();

@@ -1272,122 +1272,210 @@ __global__ __launch_bounds__(kAttnMaxRep *kWaveSize) static void attention_decod
 // ops::attention_decode keeps the reference's contract (include/ops/attention_decode.cuh:98-109):
 // no workspace and no allocation, any head_dim <= 64, q and caches at any 4-byte alignment, any
 // kv_rep, and num_q_heads need not be a multiple of kv_rep (q head h reads kv head h / kv_rep).
-// With no scratch there is nowhere to leave split-KV records, so one workgroup owns a q head, as
-// in the reference's grid. Its kSingleWaves waves take kSingleKeys-key chunks round robin, each
-// wave with its own online-softmax state (m, l, unnormalised acc), and the wave states are merged
-// in wave order at the end. A chunk is a contiguous run of n * D floats of the cache: K and V are
-// read together with coalesced 4-byte buffer loads (one memory round trip per chunk; lanes past
-// the chunk read zeros from the descriptor's range check) and staged in the wave's own LDS rows
-// of kAttnMaxD + 1 floats, an odd stride, so the lane = key reads of the score loop hit distinct
-// banks. Scores are the d-ascending fmaf chain of the reference's dot product; P V (lane = d) is
-// key-ascending within a chunk.
+// With no scratch there is nowhere to leave split-KV records, so a workgroup reads every key of its
+// q head and keeps the scores in LDS (kAttnDecodeMaxLen of them). It is bound by one CU's share of
+// the cache bandwidth and by the VALU: 16 waves read 16 bytes a lane with several rows in flight, and
+// where the heads leave CUs idle a head runs as kGK / kGV workgroups that compute the same scores and
+// take a slice of the output columns, i.e. of V, each.
+// A row (key) is kGK lanes of kV floats (kV = 4, or 1 where head_dim is no multiple of 4), so a
+// wave reads kWaveSize / kGK consecutive rows per load, and of a V slice kWaveSize / kGV rows.
+// Scores: an fmaf chain over a lane's floats, summed over the row's lanes; one maximum and one sum
+// over the workgroup; P V in row order per lane, lanes and waves summed at the end.
 // Workgroup b serves q head (b % 8) * (qh / 8) + b / 8 when 8 divides qh: under the round-robin
 // dispatch of workgroups to the 8 XCDs, consecutive q heads, which share a kv head, then run on
 // one XCD and read their K/V through the same L2.
-constexpr int kSingleWaves = 8;
-constexpr int kSingleKeys = 32;
-constexpr int kSingleStride = kAttnMaxD + 1;
-constexpr int kSinglePer = kSingleKeys * kAttnMaxD / kWaveSize; // chunk floats per lane at most
+constexpr int kSingleWaves = 16;
+constexpr int kSingleAhead = 4; // rows per lane in a batch; one batch is in flight while one is used
 
-__global__ __launch_bounds__(kSingleWaves *kWaveSize) static void attention_decode_single_kernel(
+// Sum over each aligned group of kG lanes, in every lane of the group.
+template <int kG> __device__ __forceinline__ float lane_group_sum(float v) {
+    if constexpr (kG >= 2)
+        v += wave::dpp<wave::kQuadSwap1>(v, v);
+    if constexpr (kG >= 4)
+        v += wave::dpp<wave::kQuadSwap2>(v, v);
+    if constexpr (kG >= 8)
+        v += wave::dpp<wave::kRowHalfMirror>(v, v);
+    if constexpr (kG >= 16)
+        v += wave::dpp<wave::kRowMirror>(v, v);
+    if constexpr (kG >= 32)
+        v += __shfl_xor(v, 16);
+    if constexpr (kG >= 64)
+        v += __shfl_xor(v, 32);
+    return v;
+}
+
+// The rows of one wave in order, kRows per load: row0 = kRows * wave, then every
+// kSingleWaves * kRows. start() issues the first batch; run() calls use(row, pack) per lane and
+// row, with use(row, pack, false) where the lane's row may lie past len (it then holds row len - 1).
+template <int kV, int kRows> struct SingleStream {
+    using Pack = float __attribute__((ext_vector_type(kV)));
+    using PackU = Pack __attribute__((aligned(4)));
+    static constexpr int kStep = kSingleWaves * kRows, kBatch = kStep * kSingleAhead;
+    const float *base; // row 0
+    int D, len, row0, sub, col;
+    Pack buf[2][kSingleAhead];
+
+    __device__ __forceinline__ void load(Pack (&p)[kSingleAhead], int r) const {
+        if (r + kBatch <= len) { // one lane offset for the batch, the rest in scalar registers
+#pragma unroll
+            for (int i = 0; i < kSingleAhead; ++i)
+                p[i] = *reinterpret_cast<const PackU *>(base + (r + kStep * i) * D + (sub * D + col));
+        } else {
+#pragma unroll
+            for (int i = 0; i < kSingleAhead; ++i) {
+                const int row = r + sub + kStep * i;
+                p[i] = *reinterpret_cast<const PackU *>(base + (row < len ? row : len - 1) * D + col);
+            }
+        }
+    }
+    __device__ __forceinline__ void start() {
+        if (row0 < len)
+            load(buf[0], row0);
+    }
+    template <typename Use> __device__ __forceinline__ void run(Use &&use) {
+        auto consume = [&](const Pack (&p)[kSingleAhead], int r, auto whole) {
+#pragma unroll
+            for (int i = 0; i < kSingleAhead; ++i) {
+                const int row = r + sub + kStep * i;
+                use(row, p[i], decltype(whole)::value || row < len);
+            }
+        };
+        // Every batch but the last is whole. The exits are separate copies, so no join of paths with
+        // different loads in flight makes the loop wait for all of them.
+        for (int r = row0; r < len; r += 2 * kBatch) {
+            if (r + kBatch >= len) {
+                consume(buf[0], r, std::false_type{});
+                return;
+            }
+            load(buf[1], r + kBatch);
+            consume(buf[0], r, std::true_type{});
+            if (r + 2 * kBatch >= len) {
+                consume(buf[1], r + kBatch, std::false_type{});
+                return;
+            }
+            load(buf[0], r + 2 * kBatch);
+            consume(buf[1], r + kBatch, std::true_type{});
+        }
+    }
+};
+
+template <int kV, int kGK, int kGV>
+__global__ __launch_bounds__(kSingleWaves *kWaveSize) void attention_decode_single_kernel(
     const float *__restrict__ q, const float *__restrict__ kcache, const float *__restrict__ vcache,
     float *__restrict__ out, int num_q_heads, int kv_rep, int D, int len, int max_seq, float scale) {
-    __shared__ float Qs[kAttnMaxD];
-    __shared__ float Ks[kSingleWaves][kSingleKeys * kSingleStride];
-    __shared__ float Vs[kSingleWaves][kSingleKeys * kSingleStride];
-    __shared__ float Ps[kSingleWaves][kSingleKeys];
+    constexpr int kSlices = kGK / kGV, kRowsK = kWaveSize / kGK, kRowsV = kWaveSize / kGV;
+    __shared__ float Ss[kAttnDecodeMaxLen];
+    __shared__ float Wacc[kSingleWaves][kV * kGV];
     __shared__ float Wm[kSingleWaves], Wl[kSingleWaves];
-    __shared__ float Wacc[kSingleWaves][kAttnMaxD];
-    const int b = blockIdx.x;
+    const int b = blockIdx.x / kSlices, slice = blockIdx.x % kSlices;
     const int h = num_q_heads % 8 == 0 ? (b % 8) * (num_q_heads / 8) + b / 8 : b;
-    const int wave = threadIdx.x / kWaveSize, lane = threadIdx.x % kWaveSize;
+    const int lane = threadIdx.x % kWaveSize;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWaveSize);
     const int64_t kv_base = int64_t(h / kv_rep) * max_seq * D;
-    if (threadIdx.x < D)
-        Qs[threadIdx.x] = q[int64_t(h) * D + threadIdx.x];
-    __syncthreads();
-    // element e = lane + 64 i of a chunk is key e / D, dimension e % D; stepped without division
-    const int key0 = lane / D, d0 = lane % D, key_step = kWaveSize / D, d_step = kWaveSize % D;
-    const int per = (kSingleKeys * D + kWaveSize - 1) / kWaveSize; // loads per lane per chunk
-    float *ks = Ks[wave], *vs = Vs[wave];
-    float m = kNegInf, l = 0.f, acc = 0.f;
-    for (int c0 = wave * kSingleKeys; c0 < len; c0 += kSingleWaves * kSingleKeys) {
-        const int n = len - c0 < kSingleKeys ? len - c0 : kSingleKeys;
-        const int64_t off = kv_base + int64_t(c0) * D;
-        const __amdgpu_buffer_rsrc_t ksrc = operand_rsrc(kcache + off, int64_t(n) * D * 4);
-        const __amdgpu_buffer_rsrc_t vsrc = operand_rsrc(vcache + off, int64_t(n) * D * 4);
-        float kr[kSinglePer], vr[kSinglePer];
+    // Lanes past the row's end (D < kV kGK) read its last pack again and count for nothing.
+    const int kcol = kV * (lane % kGK), vcol = kV * kGV * slice + kV * (lane % kGV);
+    const bool kin = kcol < D, vin = vcol < D;
+    SingleStream<kV, kRowsK> ks{kcache + kv_base, D, len, kRowsK * wave, lane / kGK, kin ? kcol : D - kV, {}};
+    SingleStream<kV, kRowsV> vs{vcache + kv_base, D, len, kRowsV * wave, lane / kGV, vin ? vcol : D - kV, {}};
+    ks.start();
+    float qv[kV];
 #pragma unroll
-        for (int i = 0; i < kSinglePer; ++i) {
-            if (i < per) {
-                kr[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ksrc, 4 * lane, 4 * kWaveSize * i, 0));
-                vr[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(vsrc, 4 * lane, 4 * kWaveSize * i, 0));
-            }
-        }
-        {
-            int key = key0, d = d0;
-#pragma unroll
-            for (int i = 0; i < kSinglePer; ++i) {
-                if (i < per && key < n) {
-                    ks[key * kSingleStride + d] = kr[i];
-                    vs[key * kSingleStride + d] = vr[i];
-                }
-                key += key_step;
-                d += d_step;
-                if (d >= D) {
-                    d -= D;
-                    ++key;
-                }
-            }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    for (int j = 0; j < kV; ++j)
+        qv[j] = q[int64_t(h) * D + (kin ? kcol : D - kV) + j];
+    float m = kNegInf;
+    ks.run([&](int row, const auto &k, bool in) {
         float s = 0.f;
-        if (lane < n)
-            for (int d = 0; d < D; ++d)
-                s = fmaf(Qs[d], ks[lane * kSingleStride + d], s);
-        const float sc = lane < n ? s * scale : kNegInf;
-        const float mn = fmaxf(m, wave::max(sc)); // finite: the chunk has at least one key
-        const float corr = m == kNegInf ? 0.f : expf(m - mn);
-        const float p = lane < n ? expf(sc - mn) : 0.f;
-        l = l * corr + wave::sum(p);
-        m = mn;
-        if (lane < kSingleKeys)
-            Ps[wave][lane] = p;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        if (lane < D) {
-            float o = acc * corr;
-            for (int k = 0; k < n; ++k)
-                o = fmaf(Ps[wave][k], vs[k * kSingleStride + lane], o);
-            acc = o;
+#pragma unroll
+        for (int j = 0; j < kV; ++j)
+            s = fmaf(qv[j], k[j], s);
+        s = lane_group_sum<kGK>(kin ? s : 0.f);
+        if (in) {
+            m = fmaxf(m, s);
+            if (lane % kGK == 0)
+                Ss[row] = s;
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    }
-    if (lane < D)
-        Wacc[wave][lane] = acc;
-    if (lane == 0) {
+    });
+    vs.start(); // in flight over the softmax
+    m = wave::max(m);
+    if (lane == 0)
         Wm[wave] = m;
+    __syncthreads();
+    float M = Wm[0];
+#pragma unroll
+    for (int w = 1; w < kSingleWaves; ++w)
+        M = fmaxf(M, Wm[w]);
+    M *= scale; // of the scaled scores too: scaling keeps their order
+    float l = 0.f;
+    for (int i = threadIdx.x; i < len; i += kSingleWaves * kWaveSize) {
+        const float p = expf(Ss[i] * scale - M);
+        Ss[i] = p;
+        l += p;
+    }
+    l = wave::sum(l);
+    if (lane == 0)
         Wl[wave] = l;
+    __syncthreads();
+    float acc[kV] = {};
+    vs.run([&](int row, const auto &v, bool in) {
+        if (in) {
+            const float p = Ss[row];
+#pragma unroll
+            for (int j = 0; j < kV; ++j)
+                acc[j] = fmaf(p, v[j], acc[j]);
+        }
+    });
+#pragma unroll
+    for (int j = 0; j < kV; ++j) {
+#pragma unroll
+        for (int o = kGV; o < kWaveSize; o *= 2)
+            acc[j] += __shfl_xor(acc[j], o);
+        if (lane < kGV)
+            Wacc[wave][kV * lane + j] = acc[j];
     }
     __syncthreads();
-    if (wave != 0 || lane >= D)
+    const int c = threadIdx.x, col = kV * kGV * slice + c;
+    if (c >= kV * kGV || col >= D)
         return;
-    float M = kNegInf;
-#pragma unroll
-    for (int w = 0; w < kSingleWaves; ++w)
-        M = fmaxf(M, Wm[w]);
     float L = 0.f, o = 0.f;
 #pragma unroll
     for (int w = 0; w < kSingleWaves; ++w) {
-        const float f = Wm[w] == kNegInf ? 0.f : expf(Wm[w] - M); // a wave past the length holds nothing
-        L = fmaf(Wl[w], f, L);
-        o = fmaf(Wacc[w][lane], f, o);
+        L += Wl[w];
+        o += Wacc[w][c];
     }
-    out[int64_t(h) * D + lane] = o / L;
+    out[int64_t(h) * D + col] = o / L;
+}
+
+inline void attention_decode_single_launch(const float *q, const float *kcache, const float *vcache, float *out,
+                                           int num_q_heads, int kv_rep, int D, int len, int max_seq,
+                                           hipStream_t stream) {
+    const float scale = 1.f / std::sqrt(static_cast<float>(D));
+    auto run = [&](auto v, auto gk, auto gv) {
+        constexpr int kV = decltype(v)::value, kGK = decltype(gk)::value, kGV = decltype(gv)::value;
+        launch_async(stream, attention_decode_single_kernel<kV, kGK, kGV>, num_q_heads * (kGK / kGV),
+                     kSingleWaves * kWaveSize, q, kcache, vcache, out, num_q_heads, kv_rep, D, len, max_seq, scale);
+    };
+    using std::integral_constant;
+    constexpr auto c1 = integral_constant<int, 1>{};
+    constexpr auto c4 = integral_constant<int, 4>{};
+    constexpr auto c8 = integral_constant<int, 8>{};
+    constexpr auto c16 = integral_constant<int, 16>{};
+    constexpr auto c64 = integral_constant<int, 64>{};
+    const int64_t n = int64_t(num_q_heads) * D;
+    // The slices of a head read its q while others store: out must not be q.
+    const bool apart = out + n <= q || q + n <= out;
+    const bool slices = apart && int64_t(num_q_heads) * (D / 16) <= cu_count();
+    if (D % 4 == 0) {
+        if (D > 32)
+            D == 64 && slices ? run(c4, c16, c4) : run(c4, c16, c16);
+        else if (D > 16)
+            D == 32 && slices ? run(c4, c8, c4) : run(c4, c8, c8);
+        else
+            run(c4, c4, c4);
+    } else if (D > 16) {
+        run(c1, c64, c64);
+    } else {
+        run(c1, c16, c16);
+    }
 }
 
 // Enqueues the partial and combine kernels (or the fused partial kernel alone
@@ -1600,9 +1688,8 @@ inline void attention_decode(const float *q, const float *kcache, const float *v
     detail::require(len > 0 && len <= max_seq, "attention_decode: len must be in [1, max_seq]");
     detail::require(len <= detail::kAttnDecodeMaxLen, "attention_decode: len must be at most 8192");
     detail::require(q && kcache && vcache && out, "attention_decode: null pointer");
-    const float scale = 1.f / std::sqrt(static_cast<float>(head_dim));
-    launch_async(stream, detail::attention_decode_single_kernel, num_q_heads, detail::kSingleWaves * kWaveSize,
-                         q, kcache, vcache, out, num_q_heads, kv_rep, head_dim, len, max_seq, scale);
+    detail::attention_decode_single_launch(q, kcache, vcache, out, num_q_heads, kv_rep, head_dim, len, max_seq,
+                                           stream);
 }
 
 } // namespace opworks::ops

@@ -1,0 +1,46 @@
+"""The scratch-free decode attention at the edges of its layouts: one workgroup per q head or one per slice
+of a head's output, and lengths around its 64- to 512-row batches. Against numpy in float64.
+
+Tolerance: a score is an fmaf chain of at most 4 terms and 6 pairwise sums (10 roundings, and the scaling),
+which the softmax turns into a relative error of its size; p and its sum add a few ulp of expf and a chain of
+at most len / 1024 terms; P V is a chain of at most len / 16 terms and 8 pairwise sums. So
+|got - want| <= 2^-24 (2 (12 max|score| + 16) + len / 16 + 32) * sum p |v|."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(ow, heads, kv_rep, dim, length, in_place):
+    rng = np.random.default_rng(heads * 1000003 + dim * 1009 + length)
+    kvh, cap = -(-heads // kv_rep), length + 2
+    q = rng.standard_normal((heads, dim)).astype(np.float32)
+    k, v = (rng.standard_normal((kvh, cap, dim)).astype(np.float32) for _ in range(2))
+    k[:, length:], v[:, length:] = np.nan, np.nan
+    dq, dk, dv = (ow.DeviceBuffer.from_host(a.reshape(-1)) for a in (q, k, v))
+    out = dq if in_place else ow.DeviceBuffer.empty(heads * dim)
+    ow.ops.attention_decode(dq, dk, dv, out, heads, kv_rep, dim, length, cap)
+    got = out.to_host().reshape(heads, dim)
+    kh = np.repeat(k[:, :length].astype(np.float64), kv_rep, 0)[:heads]
+    vh = np.repeat(v[:, :length].astype(np.float64), kv_rep, 0)[:heads]
+    s = np.einsum("hd,hnd->hn", q.astype(np.float64), kh) / np.sqrt(dim)
+    size = np.einsum("hd,hnd->hn", np.abs(q), np.abs(kh)).max(1, keepdims=True) / np.sqrt(dim)
+    p = np.exp(s - s.max(1, keepdims=True))
+    p /= p.sum(1, keepdims=True)
+    want, bound = np.einsum("hn,hnd->hd", p, vh), np.einsum("hn,hnd->hd", p, np.abs(vh))
+    tol = 2.0 ** -24 * (2 * (12 * size + 16) + length / 16 + 32) * bound
+    assert np.all(np.abs(got - want) <= tol), float(np.max(np.abs(got - want) / tol))
+
+
+# 64 and 32 columns run in slices up to 64 and 128 heads; 16, 20 and 48 never do
+@pytest.mark.parametrize("heads,kv_rep,dim", [(8, 4, 64), (64, 8, 64), (65, 4, 64), (128, 16, 32), (129, 16, 32),
+                                              (16, 1, 32), (8, 2, 16), (4, 2, 20), (3, 3, 48), (4, 4, 62)])
+@pytest.mark.parametrize("length", [1, 63, 64, 255, 256, 257, 511, 513, 1025, 2047])
+def test_decode_single(ow, heads, kv_rep, dim, length):
+    _case(ow, heads, kv_rep, dim, length, False)
+
+
+@pytest.mark.parametrize("heads,kv_rep,dim", [(8, 4, 64), (16, 1, 32), (4, 2, 20)])
+def test_decode_single_in_place(ow, heads, kv_rep, dim):
+    """The output over q: a head then runs as one workgroup, which has read its q before it stores."""
+    _case(ow, heads, kv_rep, dim, 700, True)
