@@ -125,7 +125,7 @@ inline void layer_norm(const float *in, float *out, const float *gamma, const fl
     detail::require(in && out && gamma && beta, "layer norm requires non-null pointers");
     const bool packed = detail::aligned16(in) && detail::aligned16(out) && detail::aligned16(gamma) &&
                         detail::aligned16(beta);
-    const detail::RowPlan plan = detail::plan_row(cols);
+    const detail::RowPlan plan = detail::plan_row_for_rows(rows, cols);
     if (plan.waves == 0 && detail::row_split_ok(in, out, rows, cols)) {
         detail::row_split_launch<detail::LayerNormSplit>(in, out, gamma, beta, rows, cols, eps, stream);
         return;
@@ -134,7 +134,7 @@ inline void layer_norm(const float *in, float *out, const float *gamma, const fl
         launch_async(stream, detail::layer_norm_stream_kernel, rows, kThreads, in, out, gamma, beta, cols, eps);
         return;
     }
-    detail::dispatch_row_plan(plan, [&](auto w, auto v) {
+    detail::dispatch_row_plan_for_rows(plan, [&](auto w, auto v) {
         constexpr int kW = decltype(w)::value, kV = decltype(v)::value;
         detail::dispatch_row_fit(detail::row_fit<kW, kV>(cols, packed), [&](auto fit) {
             launch_async(stream, detail::layer_norm_reg_kernel<kW, kV, decltype(fit)::value>,

@@ -170,13 +170,15 @@ inline RowPlan plan_row(int cols) {
     return {16, 8};
 }
 
-// The plan for `rows` rows: a short matrix (fewer than 2048 row waves, 8 per CU) spreads each
+// The plan for `rows` rows: a short matrix (fewer than 4096 row waves, 16 per CU) spreads each
 // row over more waves with fewer packs each, down to 2 packs per lane, so the GPU has enough
-// waves in flight: 512 x 2048 (a 512-token prefill's RMSNorm) runs 4 waves of 2 packs per row
-// instead of 1 wave of 8. Only the row ops whose dispatch carries these shapes use it.
+// loads in flight: 512 x 2048 (a 512-token prefill's RMSNorm) runs 4 waves of 2 packs per row
+// instead of 1 wave of 8. LayerNorm and softmax of 1500 x 2048, 1 -> 4 waves a row: 4.9 -> 4.0
+// and 4.5 -> 4.2 us; 3000 x 2048, 1 -> 2: 8.3 -> 7.3 and 6.7 -> 6.0. With the line at 2048 the latter
+// stays at one wave (8.4 and 6.6), at 8192 its 4 waves cost more than they hide (8.6 and 7.6).
 inline RowPlan plan_row_for_rows(int rows, int cols) {
     RowPlan p = plan_row(cols);
-    while (p.waves != 0 && p.packs >= 4 && p.waves <= 4 && int64_t(rows) * p.waves < 2048) {
+    while (p.waves != 0 && p.packs >= 4 && p.waves <= 4 && int64_t(rows) * p.waves < 4096) {
         p.waves *= 2;
         p.packs /= 2;
     }
@@ -201,7 +203,7 @@ template <typename Fn> inline void dispatch_row_plan(const RowPlan &plan, Fn &&f
     }
 }
 
-// dispatch_row_plan plus the shapes plan_row_for_rows can add.
+// dispatch_row_plan plus the shapes plan_row_for_rows adds.
 template <typename Fn> inline void dispatch_row_plan_for_rows(const RowPlan &plan, Fn &&fn) {
     switch (plan.waves * 100 + plan.packs) {
     case 202: fn(IntTag<2>{}, IntTag<2>{}); break;

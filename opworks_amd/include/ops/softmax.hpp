@@ -81,7 +81,7 @@ inline void softmax(const float *in, float *out, int rows, int cols, hipStream_t
     detail::require(cols > 0, "softmax requires positive columns for nonempty rows");
     detail::require(in && out, "softmax requires non-null pointers");
     const bool packed = detail::aligned16(in) && detail::aligned16(out);
-    const detail::RowPlan plan = detail::plan_row(cols);
+    const detail::RowPlan plan = detail::plan_row_for_rows(rows, cols);
     if (plan.waves == 0 && detail::row_split_ok(in, out, rows, cols)) {
         detail::row_split_launch<detail::SoftmaxSplit>(in, out, nullptr, nullptr, rows, cols, 0.f, stream);
         return;
@@ -90,7 +90,7 @@ inline void softmax(const float *in, float *out, int rows, int cols, hipStream_t
         launch_async(stream, detail::softmax_rows_stream_kernel, rows, kThreads, in, out, cols);
         return;
     }
-    detail::dispatch_row_plan(plan, [&](auto w, auto v) {
+    detail::dispatch_row_plan_for_rows(plan, [&](auto w, auto v) {
         constexpr int kW = decltype(w)::value, kV = decltype(v)::value;
         detail::dispatch_row_fit(detail::row_fit<kW, kV>(cols, packed), [&](auto fit) {
             launch_async(stream, detail::softmax_rows_reg_kernel<kW, kV, decltype(fit)::value>,

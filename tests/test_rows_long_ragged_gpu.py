@@ -88,3 +88,14 @@ def test_softmax_special_values(ow, cols):
     assert np.all(got[0, : cols - 3] == 0) and np.all(np.isnan(got[1:4]))
     keep = [0, 4]
     _close("softmax", got[keep], _want("softmax", x[keep], g, b))
+
+
+@pytest.mark.parametrize("op", OPS)
+@pytest.mark.parametrize("rows,cols", [
+    (1, 1024), (2047, 1024), (2048, 1024), (4095, 1024), (4096, 1024),   # 4 packs: 4 x 2, 2 x 2 ... 1 x 4
+    (500, 2048), (1023, 2048), (1024, 2044), (2049, 2047), (4096, 2048),  # 8 packs, whole, bounded and ragged
+    (511, 8192), (512, 8189), (1024, 8192), (70, 16380)])                 # 4 and 8 waves to begin with
+def test_short_matrices(ow, op, rows, cols):
+    """Rows spread over more waves where the matrix is short, on both sides of the line."""
+    x, g, b = _inputs(rows, cols, 2.0)
+    _close(op, _run(ow, op, x, g, b), _want(op, x, g, b))
