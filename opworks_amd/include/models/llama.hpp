@@ -768,10 +768,7 @@ template <typename WT> class LlamaModelT final : public LlamaRuntime {
                     st, reduce);
             }
         }
-        if constexpr (kBf16 && kSplittable) { // (no hook: the reduction kernel stores, the caller norms)
-            detail::gemm_bf16_launch_splitk<float, IdentityEpilogue, kStore>(
-                A, Wb, nullptr, C, M, N, K, IdentityEpilogue{}, s.workspace.splitk.data(), s.workspace.splitk.size(), st);
-        } else if constexpr (kBf16) {
+        if constexpr (kBf16) { // (no hook: the caller norms)
             detail::gemm_bf16_launch<float, IdentityEpilogue, kStore>(A, Wb, nullptr, C, M, N, K, IdentityEpilogue{},
                                                                       st);
         } else if constexpr (kSplittable) { // fp32 MFMA kernels: the oracle parity of the logits

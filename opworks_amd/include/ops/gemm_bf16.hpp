@@ -2,41 +2,20 @@
 
 // bf16 GEMM with fp32 accumulation on the CDNA4 matrix cores:
 //   C[m][n] = epi(sum_k bf16(A[m][k]) * W[n][k] + bias[n]),   W bf16 [N][K] (HF layout).
-// A is either fp32 (rounded to bf16, nearest-even, while it is staged into LDS —
-// the reference's ops::linear_mma_bf16 contract, include/ops/linear_mma.cuh:24-93)
-// or already bf16.
-//
-// Kernel shape (gfx950):
-//  * workgroup tile 256 x 256, 512 threads = 8 waves in 2 x 4; each wave owns
-//    128 x 64 outputs (128 accumulator registers);
-//  * K tile 64 (128 KB of LDS with bf16 A, 144 KB with fp32 A; one workgroup
-//    per CU);
-//  * an MFMA operand is 8 consecutive k of one row per lane, so both operands
-//    keep their k-contiguous global layout in LDS; the reads of 16
-//    consecutive rows fall on disjoint bank groups, by XOR-swizzled 16-byte
-//    chunks (chunk c of row r in slot c ^ ((r >> 1) & 7)) where loads go
-//    straight to LDS and by 16 bytes of row padding where they are staged in
-//    registers;
-//  * with bf16 A both operands go from global memory straight into LDS
-//    (gfx950 global_load_lds_dwordx4, no register staging) and the wave tile
-//    is 8 x 4 v_mfma_f32_16x16x32_bf16 tiles, two MFMA steps per K tile. The
-//    workgroup syncs once per K tile, before the last step's MFMAs, whose
-//    operands are already in registers: the next tile's first fragments are
-//    read while those MFMAs run, so no step waits on the barrier's LDS reads;
-//  * with fp32 A both operands are loaded into registers (A raw, rounded when
-//    written to LDS) and stored halfway through the current tile's MFMAs, on
-//    4 x 2 v_mfma_f32_32x32x16_bf16 tiles (the 16x16 form's fragments would
-//    not fit beside the staging registers);
-//  * LDS double buffered, the next tile's loads issued before the current
-//    tile's MFMAs; inside a tile the next MFMA step's fragments are read while
-//    the current step's MFMAs run; same XCD-banded tile order as the fp32
-//    kernel.
-// On 4096^3 uniformly random bf16 operands the 16x16x32 and 32x32x16 forms gave
-// bit-identical outputs (measured on gfx950); the tests hold both to the oracle.
-
-#include <cstddef>
-#include <cstdint>
-#include <type_traits>
+// A is either fp32 (rounded to bf16, nearest-even, as it is staged — the reference's
+// ops::linear_mma_bf16 contract, include/ops/linear_mma.cuh:24-93) or already bf16. fp32 A and operands off the
+// 16-byte grid take gemm_x6_kernel and gemm_rows_kernel with one bf16 part per value; on the grid,
+// bf16 A and W also have the direct-load kernel below (gfx950):
+//  * workgroup tiles of 128 to 256 x 256, 512 threads = 8 waves in 2 x 4, one workgroup per CU;
+//  * K tile 64, both operands straight from global memory into LDS (global_load_lds_dwordx4, no
+//    register staging) in their k-contiguous global layout: an MFMA operand is 8 consecutive k of one row per
+//    lane. The reads of 16 consecutive rows fall on disjoint bank groups by XOR-swizzled 16-byte chunks
+//    (chunk c of row r in slot c ^ ((r >> 1) & 7));
+//  * v_mfma_f32_16x16x32_bf16 tiles, two MFMA steps per K tile. The workgroup syncs once per K
+//    tile, before the last step's MFMAs, whose operands are already in registers: the next tile's first
+//    fragments are read while those MFMAs run, so no step waits on the barrier's LDS reads;
+//  * two or three LDS stages, the next tiles' loads issued before the current tile's MFMAs; the same
+//    XCD-banded tile order as the fp32 kernel.
 
 #include "../core/bf16.hpp"
 #include "../core/lds_direct.hpp"
@@ -49,68 +28,41 @@ namespace opworks::detail {
 using bf16x8 = __bf16 __attribute__((ext_vector_type(8)));
 using u32x4 = uint32_t __attribute__((ext_vector_type(4)));
 
-constexpr int kBfBM = 256, kBfBN = 256;
-constexpr int kBfBK = 32; // K granularity of split-K planning (the smaller of the two K tiles)
-constexpr int kBfThreads = 512;
+constexpr int kBfBK = 64; // K tile; against 32: 945 -> 1013-1030 TFLOP/s, 512-token TTFT 4.5 -> 4.05 ms
 
-// Products of so few rows take gemm_rows_kernel.
-constexpr int kRowsMax = 64;
-inline bool gemm_rows_use(int M, int K) { return M <= kRowsMax && K > 0; }
-
-// Workgroup tile shapes. Big: 256 x 256 outputs, 8 waves in 2 x 4 (128 x 64 each), one
-// workgroup per CU. Small: 128 x 128, 4 waves in 2 x 2 (64 x 64 each), 64 KB of LDS so two
-// workgroups share a CU; for short-M products (prefill projections at a few hundred rows), where
-// 256 x 256 tiles leave CUs idle or force deep split-K. The small shape exists on the direct
-// path only (bf16 A, 16-byte aligned operands).
+// Workgroup tile shapes, waves WM x WN. Big: 256 x 256 outputs (128 x 64 per wave), two LDS stages,
+// for products that fill the chip with them. Tall: 128 x 256, three stages (144 KB), so two K tiles are in
+// flight while one is multiplied: at 512 rows, against two 128 x 128 workgroups per CU on two stages,
+// gate/up 56-60 -> 43-45 us, and a 256 x 128 tile 57-59 us on two stages, 44-49 on three. Mid: 192 x 256, two
+// stages, for row counts whose tall tiles just miss a round (700 x 16384, K 2048: 384 tall tiles 60 us, 256
+// mid tiles 53).
 struct BfBig {
     static constexpr int BM = 256, BN = 256, kThreads = 512, WM = 2, WN = 4, kStages = 2;
 };
-struct BfSmall {
-    static constexpr int BM = 128, BN = 128, kThreads = 256, WM = 2, WN = 2, kStages = 2;
+struct BfMid {
+    static constexpr int BM = 192, BN = 256, kThreads = 512, WM = 2, WN = 4, kStages = 2;
 };
-// Tall: 128 x 256 outputs, 8 waves in 2 x 4 (64 x 64 each), three LDS stages (144 KB, one
-// workgroup per CU), so two K tiles are in flight while one is multiplied. For short-M products
-// from 256 rows (the prefill projections). At 512 rows, against two 128 x 128 workgroups per CU
-// on two stages (same outputs, bit for bit): gate/up 56-60 -> 43-45 us, down (8 splits) 28-33 ->
-// 25-26, qkv 16.0-16.2 -> 14.2-14.9, o_proj 13.9-14.3 -> 13.4-13.6. The third stage is what pays:
-// a 256 x 128 tile on two stages ran as slowly as the small tiles (57-59 us for gate/up), on three
-// 44-49 us.
 struct BfTall {
     static constexpr int BM = 128, BN = 256, kThreads = 512, WM = 2, WN = 4, kStages = 3;
 };
 
-__device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
-    return static_cast<uint32_t>(float_to_bf16_rne(lo)) | (static_cast<uint32_t>(float_to_bf16_rne(hi)) << 16);
-}
-
-template <typename TA, bool kVec, typename Epi, GemmStore kStore = GemmStore::store, typename Shape = BfBig>
-__global__ __launch_bounds__(Shape::kThreads) void gemm_bf16_mfma_kernel(const TA *__restrict__ A,
+template <typename Epi, GemmStore kStore, typename Shape>
+__global__ __launch_bounds__(Shape::kThreads) void gemm_bf16_mfma_kernel(const uint16_t *__restrict__ A,
                                                                     const uint16_t *__restrict__ W,
                                                                     const float *__restrict__ bias,
                                                                     float *__restrict__ C, int M, int N, int K,
                                                                     Epi epi) {
-    static_assert(std::is_same_v<TA, float> || std::is_same_v<TA, uint16_t>, "A is fp32 or bf16 bits");
-    constexpr bool kF32A = std::is_same_v<TA, float>;
-    constexpr int BK = 64; // against 32: 945 -> 1013-1030 TFLOP/s (bf16 A), 512-token bf16 TTFT 4.5 -> 4.05 ms
-    // Both operands go straight from global memory into LDS (gfx950 global_load_lds_dwordx4)
-    // on the vector path with bf16 A. With fp32 A, which is rounded on the way in registers,
-    // and on the scalar path both are staged through registers.
-    constexpr bool kDirect = kVec && !kF32A;
+    constexpr int BK = kBfBK;
     constexpr int kBM = Shape::BM, kBN = Shape::BN, kT = Shape::kThreads;
     constexpr int kWTM = kBM / Shape::WM, kWTN = kBN / Shape::WN; // outputs per wave
-    static_assert(std::is_same_v<Shape, BfBig> || kDirect, "the small and tall tiles run on the direct path only");
-    static_assert(kBM == kBN || kDirect, "register staging: both operands stage the same rows per thread");
     constexpr int kStages = Shape::kStages;
-    static_assert(kStages == 2 || kDirect, "register staging is double buffered");
     // LDS rows: a direct load writes 1 KB of consecutive bytes, so its rows are unpadded, with
     // chunk c of row r in slot c ^ ((r >> 1) & 7). The LDS serves 256 bytes a cycle, 16 lanes of
     // a 16-byte read, and the reads of 16 consecutive rows at one k then fall on 16 different
-    // 16-byte bank groups (with c ^ (r & 7) they fell on 8, two lanes each). Register staging
-    // pads each row by 16 bytes instead (a 144-byte stride), which does the same and keeps every
-    // read offset a compile-time constant (the swizzle took the fp32-A kernel past 256 registers).
-    constexpr int kRowE = kDirect ? BK : BK + 8;       // bf16 elements per LDS row
+    // 16-byte bank groups (with c ^ (r & 7) they fell on 8, two lanes each).
+    constexpr int kRowE = BK;                          // bf16 elements per LDS row
     constexpr int kCPR = BK / 8;                       // 16-byte chunks (8 k) per tile row
-    constexpr int kPer = kBM * kCPR / kT;              // chunks per thread of A (and of B when square)
+    constexpr int kPer = kBM * kCPR / kT;              // chunks per thread of A
     constexpr int kPerB = kBN * kCPR / kT;             // chunks per thread of B
     constexpr int kStage = (kBM + kBN) * kRowE;        // uint16 elements per stage
     __shared__ __attribute__((aligned(16))) uint16_t lds[kStages * kStage];
@@ -122,102 +74,42 @@ __global__ __launch_bounds__(Shape::kThreads) void gemm_bf16_mfma_kernel(const T
     const int tid = threadIdx.x, lane = tid % kWaveSize;
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWaveSize); // uniform: LDS targets in scalar registers
     const int wm = wave / Shape::WN, wn = wave % Shape::WN;
-    const int l32 = lane % 32, half = lane / 32;
     const int l16 = lane % 16, quad = lane / 16;
     // The compiler does not count direct loads as writes to the array: without a store it may
     // treat the array as never written and drop the reads. This one never runs (M >= 0).
-    if (kDirect && M < 0)
+    if (M < 0)
         lds[tid] = 0;
 
-    auto swz = [](int row, int chunk) {
-        return row * kRowE + ((kDirect ? chunk ^ ((row >> 1) & 7) : chunk) << 3);
-    };
+    auto swz = [](int row, int chunk) { return row * kRowE + ((chunk ^ ((row >> 1) & 7)) << 3); };
 
-    // Register staging: chunk tid + kT * i of each operand tile (kBM or kBN rows x BK k),
-    // row (tid + kT * i) / kCPR. The vector path loads unconditionally from clamped
-    // addresses into raw registers (fp32 A is rounded to bf16 only when staged): a load under
-    // a branch makes the compiler wait for every load in flight before the next one. Rows past
-    // M or N then hold copies of the last row, which only feed outputs that are not stored; the
-    // K tail is zeroed when staged.
-    using AStage = std::conditional_t<kF32A, f32x4, u32x4>;
-    constexpr int kAParts = kF32A ? 2 : 1;
-    constexpr int kPerMax = kPer > kPerB ? kPer : kPerB; // chunks i < kPer of A, i < kPerB of B
-    AStage ra[kPer][kAParts];
-    u32x4 rb[kPerB];
-    auto chunk_row = [&](int i) { return (tid + kT * i) / kCPR; };
-    auto chunk_k = [&](int i) { return ((tid + kT * i) % kCPR) * 8; };
-    auto load_chunk_bf16 = [&](const uint16_t *src, int row, int rows_total, int k) -> u32x4 {
-        uint16_t e[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-            e[j] = (row < rows_total && k + j < K) ? src[int64_t(row) * K + k + j] : uint16_t(0);
-        return u32x4{e[0] | (uint32_t(e[1]) << 16), e[2] | (uint32_t(e[3]) << 16), e[4] | (uint32_t(e[5]) << 16),
-                     e[6] | (uint32_t(e[7]) << 16)};
-    };
-    // Register loads of tile kt: operand A unless with_a is false, operand B if with_b.
-    auto global_load = [&](int kt, bool with_a, bool with_b) {
-        const int k0 = kt * BK;
+    // The partial last K tile goes through registers: chunk tid + kT * i of each operand tile (kBM or
+    // kBN rows x BK k), row (tid + kT * i) / kCPR, loaded unconditionally from clamped addresses (a load
+    // under a branch makes the compiler wait for every load in flight before the next one). Rows past
+    // M or N hold copies of the last row, which only feed outputs that are not stored; k past K is zeroed.
+    auto stage_tail = [&](int kt) {
+        constexpr int kPerMax = kPer > kPerB ? kPer : kPerB;
+        uint16_t *As = lds, *Bs = lds + kBM * kRowE;
+        u32x4 ra[kPer], rb[kPerB];
 #pragma unroll
         for (int i = 0; i < kPerMax; ++i) {
-            const int r = chunk_row(i), k = k0 + chunk_k(i);
-            if constexpr (kVec) {
-                const int ar = m0 + r < M ? m0 + r : M - 1, br = n0 + r < N ? n0 + r : N - 1;
-                const int kc = k < K ? k : K - 8;
-                if (with_a && i < kPer) {
-#pragma unroll
-                    for (int p = 0; p < kAParts; ++p)
-                        ra[i][p] = *reinterpret_cast<const AStage *>(A + int64_t(ar) * K + kc + 4 * p);
-                }
-                if (with_b && i < kPerB)
-                    rb[i] = *reinterpret_cast<const u32x4 *>(W + int64_t(br) * K + kc);
-            } else {
-                if (with_a && i < kPer) {
-                    if constexpr (kF32A) {
-#pragma unroll
-                        for (int p = 0; p < 2; ++p)
-#pragma unroll
-                            for (int j = 0; j < 4; ++j) {
-                                const int kk = k + 4 * p + j;
-                                ra[i][p][j] = (m0 + r < M && kk < K) ? A[int64_t(m0 + r) * K + kk] : 0.f;
-                            }
-                    } else {
-                        ra[i][0] = load_chunk_bf16(A, m0 + r, M, k);
-                    }
-                }
-                if (with_b && i < kPerB)
-                    rb[i] = load_chunk_bf16(W, n0 + r, N, k);
-            }
+            const int r = (tid + kT * i) / kCPR, k = kt * BK + tid % kCPR * 8, kc = k < K ? k : K - 8;
+            const int ar = m0 + r < M ? m0 + r : M - 1, br = n0 + r < N ? n0 + r : N - 1;
+            if (i < kPer)
+                ra[i] = *reinterpret_cast<const u32x4 *>(A + int64_t(ar) * K + kc);
+            if (i < kPerB)
+                rb[i] = *reinterpret_cast<const u32x4 *>(W + int64_t(br) * K + kc);
         }
-    };
-    auto lds_store = [&](int buf, int kt, bool zero_tail, bool with_a, bool with_b) {
-        uint16_t *As = lds + buf * kStage;
-        uint16_t *Bs = As + kBM * kRowE;
-        const int k0 = kt * BK;
 #pragma unroll
         for (int i = 0; i < kPerMax; ++i) {
-            const int k = k0 + chunk_k(i);
-            const int ia = i < kPer ? i : 0, ib = i < kPerB ? i : 0; // in range; unused when i is past
-            u32x4 av, bv = rb[ib];
-            if constexpr (kF32A)
-                av = u32x4{pack_bf16x2(ra[ia][0][0], ra[ia][0][1]), pack_bf16x2(ra[ia][0][2], ra[ia][0][3]),
-                           pack_bf16x2(ra[ia][1][0], ra[ia][1][1]), pack_bf16x2(ra[ia][1][2], ra[ia][1][3])};
-            else
-                av = ra[ia][0];
-            if (zero_tail) { // the partial last K tile only: k >= K contributes nothing
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    av[j] = k < K ? av[j] : 0u;
-                    bv[j] = k < K ? bv[j] : 0u;
-                }
-            }
-            const int off = swz(chunk_row(i), chunk_k(i) / 8);
-            if (with_a && i < kPer)
-                *reinterpret_cast<u32x4 *>(As + off) = av;
-            if (with_b && i < kPerB)
-                *reinterpret_cast<u32x4 *>(Bs + off) = bv;
+            const bool in = kt * BK + tid % kCPR * 8 < K;
+            const int off = swz((tid + kT * i) / kCPR, tid % kCPR);
+            if (i < kPer)
+                *reinterpret_cast<u32x4 *>(As + off) = in ? ra[i] : u32x4{0u, 0u, 0u, 0u};
+            if (i < kPerB)
+                *reinterpret_cast<u32x4 *>(Bs + off) = in ? rb[i] : u32x4{0u, 0u, 0u, 0u};
         }
     };
-    // Direct loads of tile kt (full K tiles of the vector path): the wave's instruction i
+    // Direct loads of tile kt (full K tiles): the wave's instruction i
     // writes the 1 KB block of rows 8 * wave + 8 * waves * i .. + 7, lane l at byte 16 l, i.e.
     // row r = block + l / 8, slot l % 8, which holds chunk (l % 8) ^ ((r >> 1) & 7) of that row;
     // (r >> 1) & 7 = (4 (wave & 1) + l / 16) & 7 for every i (8 * waves is a multiple of 16).
@@ -259,18 +151,15 @@ __global__ __launch_bounds__(Shape::kThreads) void gemm_bf16_mfma_kernel(const T
         }
     };
 
-    // Accumulators: 16x16 tiles (4 registers each) on the direct path, 32x32 tiles (16) otherwise.
-    constexpr int kTile = kDirect ? 16 : 32;
-    constexpr int FM = kWTM / kTile, FN = kWTN / kTile;
-    using Acc = std::conditional_t<kDirect, f32x4, f32x16>;
-    Acc acc[FM][FN];
+    constexpr int FM = kWTM / 16, FN = kWTN / 16;
+    f32x4 acc[FM][FN];
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
         for (int j = 0; j < FN; ++j)
-            acc[i][j] = Acc{};
+            acc[i][j] = f32x4{};
 
-    // Direct path, 16x16x32 MFMAs: fragment set p holds step s's operands, lane l reading row
+    // 16x16x32 MFMAs: fragment set p holds step s's operands, lane l reading row
     // l % 16 of each 16-row tile at k 32 s + 8 (l / 16) .. + 7 (chunk 4 s + l / 16).
     bf16x8 fa[2][FM], fb[2][FN];
     auto read16 = [&](int buf, int s, int p) {
@@ -287,13 +176,11 @@ __global__ __launch_bounds__(Shape::kThreads) void gemm_bf16_mfma_kernel(const T
                                                        Bs + swz(wn * kWTN + bn * 16 + l16, ch)));
     };
     auto mfma16 = [&](int p) {
-        if constexpr (kDirect) {
 #pragma unroll
-            for (int bm = 0; bm < FM; ++bm)
+        for (int bm = 0; bm < FM; ++bm)
 #pragma unroll
-                for (int bn = 0; bn < FN; ++bn)
-                    acc[bm][bn] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[p][bm], fb[p][bn], acc[bm][bn], 0, 0, 0);
-        }
+            for (int bn = 0; bn < FN; ++bn)
+                acc[bm][bn] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[p][bm], fb[p][bn], acc[bm][bn], 0, 0, 0);
     };
     // The fragment reads issued with a step (FM + FN of them) go one per MFMA at its start.
     auto interleave16 = [] {
@@ -305,70 +192,14 @@ __global__ __launch_bounds__(Shape::kThreads) void gemm_bf16_mfma_kernel(const T
         __builtin_amdgcn_sched_group_barrier(0x008, FM * FN - FM - FN, 0);
     };
 
-    // One K tile of the register-staged paths: BK / 16 MFMA steps on 32x32x16 tiles. The
-    // fragments are double buffered across steps: the next step's six reads are interleaved
-    // one per MFMA with the current step's first six MFMAs, so they arrive while the matrix
-    // core runs. stage_next() (the next tile's LDS stores, into the other buffer) runs halfway,
-    // so its wait for the global loads and its LDS writes overlap the second half's MFMAs
-    // (against staging after the last step: 990-999 -> 1019-1025 TFLOP/s).
-    auto compute = [&](int buf, auto &&stage_next) {
-        const uint16_t *As = lds + buf * kStage;
-        const uint16_t *Bs = As + kBM * kRowE;
-        constexpr int kSteps = BK / 16;
-        bf16x8 a[2][4], b[2][2];
-        auto read = [&](int s, bf16x8 (&fa)[4], bf16x8 (&fb)[2]) {
-            const int ch = 2 * s + half; // k 16 s + 8 half .. + 7
-#pragma unroll
-            for (int bm = 0; bm < 4; ++bm)
-                fa[bm] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4 *>(
-                                                        As + swz(wm * kWTM + bm * 32 + l32, ch)));
-#pragma unroll
-            for (int bn = 0; bn < 2; ++bn)
-                fb[bn] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4 *>(
-                                                        Bs + swz(wn * kWTN + bn * 32 + l32, ch)));
-        };
-        read(0, a[0], b[0]);
-#pragma unroll
-        for (int s = 0; s < kSteps; ++s) {
-            if (s + 1 < kSteps)
-                read(s + 1, a[(s + 1) & 1], b[(s + 1) & 1]);
-            if (s == kSteps / 2)
-                stage_next();
-            if constexpr (!kDirect) {
-#pragma unroll
-                for (int bm = 0; bm < 4; ++bm)
-#pragma unroll
-                    for (int bn = 0; bn < 2; ++bn)
-                        acc[bm][bn] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[s & 1][bm], b[s & 1][bn],
-                                                                              acc[bm][bn], 0, 0, 0);
-            }
-        }
-        __builtin_amdgcn_sched_group_barrier(0x100, 6, 0); // step 0's reads
-#pragma unroll
-        for (int s = 0; s < kSteps; ++s) {
-            if (s + 1 < kSteps) {
-#pragma unroll
-                for (int j = 0; j < 6; ++j) {
-                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0); // one of step s + 1's reads
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0); // one of step s's MFMAs
-                }
-                __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-            } else {
-                __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
-            }
-        }
-    };
-
     // K tiles of this workgroup: all of them, or split blockIdx.y's contiguous share
     const int ktiles_all = (K + BK - 1) / BK;
     const int per_split = (ktiles_all + gridDim.y - 1) / gridDim.y;
     const int kt_begin = blockIdx.y * per_split;
     const int kt_end = kt_begin + per_split < ktiles_all ? kt_begin + per_split : ktiles_all;
-    // The vector path pipelines its full K tiles and runs a partial last tile (K not a multiple
-    // of the K tile) after the loop, with the tail zeroed; the scalar path bounds every element.
-    const int kt_full = kVec ? (K / BK < kt_end ? (K / BK > kt_begin ? K / BK : kt_begin) : kt_end) : kt_end;
-    if constexpr (kDirect) {
-      if (kt_begin < kt_full) {
+    // The full K tiles are pipelined; a partial last one (K not a multiple of BK) runs after the loop.
+    const int kt_full = K / BK < kt_end ? (K / BK > kt_begin ? K / BK : kt_begin) : kt_end;
+    if (kt_begin < kt_full) {
         // Per K tile: the next tile's direct loads into the idle stage, step 0's MFMAs with step
         // 1's fragments read in between, then (every wave's loads landed, every read of this tile
         // done) one barrier, and step 1's MFMAs with the next tile's step-0 fragments read in
@@ -407,45 +238,24 @@ __global__ __launch_bounds__(Shape::kThreads) void gemm_bf16_mfma_kernel(const T
         }
         if constexpr (kInFlight > 0) // the reloads past the end land before the stages are reused
             __builtin_amdgcn_s_waitcnt(kWaitVmcnt0Only);
-      }
-    } else if (kt_begin < kt_full) {
-        // Each K tile: the next tile's loads are issued first into registers, stored halfway
-        // through the MFMA steps, then the workgroup syncs once.
-        global_load(kt_begin, true, true);
-        lds_store(0, kt_begin, false, true, true);
-        __syncthreads();
-        for (int kt = kt_begin; kt < kt_full; ++kt) {
-            const int buf = (kt - kt_begin) & 1;
-            const int next = kt + 1 < kt_full ? kt + 1 : kt;
-            global_load(next, true, true);
-            __builtin_amdgcn_sched_barrier(0);
-            compute(buf, [&] { lds_store(buf ^ 1, next, false, true, true); });
-            __syncthreads();
-        }
     }
-    if (kt_full < kt_end) { // the partial last K tile (vector path), staged through registers
-        __syncthreads(); // every wave is done with the stages (the direct path's last reads)
-        global_load(kt_full, true, true);
-        lds_store(0, kt_full, true, true, true);
+    if (kt_full < kt_end) {
+        __syncthreads(); // every wave is done with the stages
+        stage_tail(kt_full);
         __syncthreads();
-        if constexpr (kDirect) {
-            read16(0, 0, 0);
-            read16(0, 1, 1);
-            mfma16(0);
-            mfma16(1);
-        } else {
-            compute(0, [] {});
-        }
+        read16(0, 0, 0);
+        read16(0, 1, 1);
+        mfma16(0);
+        mfma16(1);
     }
     if constexpr (kStore == GemmStore::partial)
         C += int64_t(blockIdx.y) * M * N;
 
-    // Accumulator register r of a 16x16 tile holds row 4 (l / 16) + r, column l % 16; of a 32x32
-    // tile, row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32. A tile inside C on both axes stores
+    // Accumulator register r of a tile holds row 4 (l / 16) + r, column l % 16. A tile inside C on both axes stores
     // without bounds tests (each test compiled to an exec-mask branch per store).
     auto store_tile = [&](auto checked_t) {
         constexpr bool checked = decltype(checked_t)::value;
-        constexpr int kRegs = kDirect ? 4 : 16; // accumulator registers per tile
+        constexpr int kRegs = 4; // accumulator registers per tile
         // A store counts in vmcnt like a load, so a load issued after stores waits for them too:
         // every bias value is loaded before the first store, and the residual C values of a
         // batch of tiles before its stores (one drain per batch, not one per element).
@@ -456,20 +266,17 @@ __global__ __launch_bounds__(Shape::kThreads) void gemm_bf16_mfma_kernel(const T
         if (kStore != GemmStore::partial && bias != nullptr) { // one uniform test for every column
 #pragma unroll
             for (int bn = 0; bn < FN; ++bn) {
-                const int col = n0 + wn * kWTN + bn * kTile + (kDirect ? l16 : l32);
+                const int col = n0 + wn * kWTN + bn * 16 + l16;
                 bv[bn] = (!checked || col < N) ? bias[col] : 0.f;
             }
         }
-        auto row_of = [&](int bm, int r) {
-            return kDirect ? m0 + wm * kWTM + bm * 16 + 4 * quad + r
-                           : m0 + wm * kWTM + bm * 32 + 8 * (r / 4) + 4 * half + (r % 4);
-        };
-        // residual loads per batch of 16 values: four 16x16 tiles or one 32x32 tile (larger batches
-        // pushed both paths into spills)
-        constexpr int kBatch = kDirect ? 4 : 1;
+        auto row_of = [&](int bm, int r) { return m0 + wm * kWTM + bm * 16 + 4 * quad + r; };
+        // residual loads per batch of 12 or 16 values (larger batches spilled)
+        constexpr int kBatch = FM % 4 == 0 ? 4 : 3;
+        static_assert(FM % kBatch == 0, "whole batches");
 #pragma unroll
         for (int bn = 0; bn < FN; ++bn) {
-            const int col = n0 + wn * kWTN + bn * kTile + (kDirect ? l16 : l32);
+            const int col = n0 + wn * kWTN + bn * 16 + l16;
             const bool col_ok = !checked || col < N;
 #pragma unroll
             for (int bm0 = 0; bm0 < FM; bm0 += kBatch) {
@@ -518,123 +325,121 @@ __global__ __launch_bounds__(Shape::kThreads) void gemm_bf16_mfma_kernel(const T
             }
         }
     };
-    // The register-staged paths keep the checked form only: a second copy pushed them into spills.
-    if constexpr (kDirect) {
-        if (m0 + kBM <= M && n0 + kBN <= N)
-            store_tile(std::false_type{});
-        else
-            store_tile(std::true_type{});
-    } else {
-        store_tile(std::true_type{});
-    }
-}
-
-// C written per kStore (see GemmStore): store, += (residual), or SwiGLU of
-// interleaved (gate, up) column pairs into C[M][N / 2]. Up to 64 rows take gemm_rows_kernel.
-template <typename TA, typename Epi, GemmStore kStore = GemmStore::store>
-void gemm_bf16_launch(const TA *A, const uint16_t *W, const float *bias, float *C, int M, int N, int K, Epi epi,
-                      hipStream_t stream, int splits = 1) {
-    require((kStore != GemmStore::swiglu && kStore != GemmStore::swiglu_bf16) || N % 2 == 0,
-            "swiglu epilogue needs an even number of columns");
-    if constexpr (kStore != GemmStore::partial) {
-        if (splits == 1 && gemm_rows_use(M, K)) {
-            constexpr bool kRound = std::is_same_v<TA, float>;
-            const GemmPick pick = gemm_pick(kGemmCostWbf16, M, N, K, false, gemm_rows_staged_ok<BLayout::nk>(A, W, N, K));
-            gemm_tile_launch<BLayout::nk, kRound, Epi, kStore>(pick.tile, A, W, bias, C, M, N, K, epi, stream);
-            return;
-        }
-    }
-    const int tiles = static_cast<int>(blocks_for64(M, kBfBM) * blocks_for64(N, kBfBN));
-    const dim3 grid(tiles, splits);
-    const bool vec = aligned16(A) && aligned16(W) && K % 8 == 0;
-    if (vec)
-        launch_async(stream, gemm_bf16_mfma_kernel<TA, true, Epi, kStore>, grid, kBfThreads, A, W, bias, C, M, N, K,
-                     epi);
+    if (m0 + kBM <= M && n0 + kBN <= N)
+        store_tile(std::false_type{});
     else
-        launch_async(stream, gemm_bf16_mfma_kernel<TA, false, Epi, kStore>, grid, kBfThreads, A, W, bias, C, M, N, K,
-                     epi);
+        store_tile(std::true_type{});
 }
 
-// Floats of split-K workspace any launch planned by splitk_factor(tiles, ., 256) needs (the
-// small- and tall-tile plans below stay within it: splits x tiles <= 512 tiles of a quarter the
-// size, or <= 256 of half).
-constexpr int64_t kSplitKWorkspaceBf16 = int64_t(256) * kBfBM * kBfBN;
+// Whether bf16 operands can take the direct-load tiles: whole 16-byte chunks of every row.
+inline bool gemm_bf16_direct_ok(const uint16_t *A, const uint16_t *W, int K) {
+    return aligned16(A) && aligned16(W) && K % 8 == 0 && K > 0;
+}
 
-// Split-K form of gemm_bf16_launch for store / residual outputs (see
-// gemm_f32_launch_splitk); 256-wide tiles, so one round of 256 workgroups.
+// C written per kStore (see GemmStore): store, += (residual), or SwiGLU of interleaved (gate, up)
+// column pairs into C[M][N / 2]. A is fp32, rounded as it is staged, or bf16 at any alignment.
 template <typename TA, typename Epi, GemmStore kStore>
-void gemm_bf16_launch_splitk(const TA *A, const uint16_t *W, const float *bias, float *C, int M, int N, int K,
-                             Epi epi, float *ws, int64_t ws_floats, hipStream_t stream) {
-    const int tiles = static_cast<int>(blocks_for64(M, kBfBM) * blocks_for64(N, kBfBN));
-    const int splits = splitk_factor(tiles, static_cast<int>(blocks_for64(K, kBfBK)), 256);
-    if (splits == 1 || gemm_rows_use(M, K) || N % 4 != 0 || !ws || int64_t(splits) * M * N > ws_floats ||
-        !aligned16(C) || (bias && !aligned16(bias))) {
-        gemm_bf16_launch<TA, Epi, kStore>(A, W, bias, C, M, N, K, epi, stream);
-        return;
-    }
-    gemm_bf16_launch<TA, IdentityEpilogue, GemmStore::partial>(A, W, nullptr, ws, M, N, K, IdentityEpilogue{}, stream,
-                                                               splits);
-    launch_async(stream, splitk_reduce_kernel<Epi, kStore>, stream_grid(int64_t(M) * N / 4), 256, ws, splits, bias, C,
-                 M, N, epi);
+void gemm_bf16_launch(const TA *A, const uint16_t *W, const float *bias, float *C, int M, int N, int K, Epi epi,
+                      hipStream_t stream) {
+    constexpr bool kRound = std::is_same_v<TA, float>;
+    constexpr bool kParts = kStore == GemmStore::store || kStore == GemmStore::swiglu;
+    const bool parts = kParts && gemm_x6_ok<BLayout::nk>(N, K);
+    const bool staged = gemm_rows_staged_ok<BLayout::nk>(A, W, N, K);
+    const GemmPick pick = kRound ? gemm_pick(kGemmCostRound, M, N, K, parts, staged)
+                                 : gemm_pick(kGemmCostBf16, M, N, K, parts && !staged, staged);
+    gemm_tile_launch<BLayout::nk, kRound, Epi, kStore>(pick.tile, A, W, bias, C, M, N, K, epi, stream);
 }
 
-// bf16 A on the direct path (both operands straight into LDS), for any M: 256 x 256 tiles when
-// they fill the GPU's 256 CUs, else 128 x 256 three-stage tiles from 256 rows (one workgroup per
-// CU), 128 x 128 tiles below (two per CU) and gemm_rows_kernel up to 64 rows, and for store / residual outputs K split across
-// workgroups toward one round of the GPU, at least 8 K tiles of 64 per split, the partial tiles
-// summed in split order by splitk_reduce_kernel. At M = 512 (a 512-token prefill) the 256 x 256
-// tiles gave gate/up 128 workgroups and qkv, o_proj and down 8-way splits on 16-24 tiles.
-// `reduce` as in gemm_f32_launch_splitk: called as reduce(ws, splits) in place of the reduction
-// kernel when K is split (small and tall tiles only). Returns true when it was.
+// Split-K workspace: at most kMaxSplits partial tiles of a product, and never more than one round of the
+// 256 CUs' tiles of 256 x 256.
+constexpr int64_t kSplitKWorkspaceBf16 = int64_t(256) * 256 * 256;
+
+// A direct-load tile's cost: rounds of tiles, each a start and end (a) and K steps of 32, whose price
+// grows with the share of the CUs that load (c0 alone, c0 + c1 on all of them). Fits to products of
+// 70..4096 rows, N 1000..16384, K 512..8192 (us, rms 10%):
+//   512 x 16384, K 2048: tall 34, mid 52, big 47; 700 x 16384: 60, 53, 61; 4096^3: 112, 152, 107;
+//   512 x 2048, K 2048: 23, 37, 37, and 11 on the 64 x 64 tiles of gemm_rows_kernel.
+struct GemmBf16Cost {
+    int bm, bn;
+    float a, c0, c1;
+};
+inline constexpr GemmBf16Cost kGemmCostTall{BfTall::BM, BfTall::BN, 7.f, 0.30f, 0.08f};
+inline constexpr GemmBf16Cost kGemmCostMid{BfMid::BM, BfMid::BN, 8.f, 0.5f, 0.2f};
+inline constexpr GemmBf16Cost kGemmCostBig{BfBig::BM, BfBig::BN, 10.f, 0.6f, 0.17f};
+
+inline float gemm_bf16_cost(const GemmBf16Cost &t, int M, int N, int K, int splits, int cus) {
+    const int64_t tiles = blocks_for64(M, t.bm) * blocks_for64(N, t.bn) * splits;
+    const float fill = tiles < cus ? static_cast<float>(tiles) / static_cast<float>(cus) : 1.f;
+    return static_cast<float>(blocks_for64(tiles, cus)) *
+           (t.a + (t.c0 + t.c1 * fill) * static_cast<float>(K) / (32.f * static_cast<float>(splits)));
+}
+
+// bf16 A and W, any M: the cheapest of the direct-load tiles, with K split across workgroups or not,
+// and gemm_rows_kernel's. Splits (store / residual outputs with a workspace) leave at least 8 K
+// tiles each; the partial tiles are summed in split order by splitk_reduce_kernel, or by
+// reduce(ws, splits) where given. Returns whether reduce was called.
 template <typename Epi, GemmStore kStore, typename Reduce = std::nullptr_t>
 bool gemm_bf16_launch_direct(const uint16_t *A, const uint16_t *W, const float *bias, float *C, int M, int N, int K,
                              Epi epi, float *ws, int64_t ws_floats, hipStream_t stream, Reduce reduce = nullptr) {
-    const bool vec = aligned16(A) && aligned16(W) && K % 8 == 0;
-    const int big_tiles = static_cast<int>(blocks_for64(M, kBfBM) * blocks_for64(N, kBfBN));
     constexpr bool kSwiglu = kStore == GemmStore::swiglu || kStore == GemmStore::swiglu_bf16;
+    constexpr bool kHook = !std::is_same_v<Reduce, std::nullptr_t>;
     require(!kSwiglu || N % 2 == 0, "swiglu epilogue needs an even number of columns");
-    if (gemm_rows_use(M, K)) { // few rows: K is split inside the workgroups
+    if (!gemm_bf16_direct_ok(A, W, K)) {
         gemm_bf16_launch<uint16_t, Epi, kStore>(A, W, bias, C, M, N, K, epi, stream);
         return false;
     }
-    if (!vec || big_tiles >= 256) {
-        if constexpr (kSwiglu)
-            gemm_bf16_launch<uint16_t, Epi, kStore>(A, W, bias, C, M, N, K, epi, stream);
-        else
-            gemm_bf16_launch_splitk<uint16_t, Epi, kStore>(A, W, bias, C, M, N, K, epi, ws, ws_floats, stream);
+    const int cus = cu_count();
+    const bool can_split = !kSwiglu && N % 4 == 0 && ws && aligned16(C) && (!bias || aligned16(bias));
+    const GemmPick rows = gemm_pick(kGemmCostBf16, M, N, K, false, true);
+    // A hook's work runs as a pass of its own behind an unsplit residual product.
+    const float unsplit = kHook && kStore == GemmStore::residual ? 5.f : 0.f;
+    float best = rows.cost + unsplit;
+    const GemmBf16Cost *tile = nullptr;
+    int splits = 1;
+    for (const GemmBf16Cost *t : {&kGemmCostTall, &kGemmCostMid, &kGemmCostBig})
+        for (int s = 1; s <= 8; s *= 2) {
+            if (s > 1 && (!can_split || blocks_for64(K, kBfBK) / s < 8 || int64_t(s) * M * N > ws_floats))
+                break;
+            // the partial tiles' way out and back in, mostly within the caches, and a launch (with 8 for 3 a
+            // 512-token prefill left the splits and took 2470 instead of 2300 us)
+            const float sum = s == 1 ? unsplit
+                                     : (kHook ? 0.f : 3.f) + static_cast<float>(int64_t(s) * M * N) * (3.f / 6e6f);
+            const float cost = gemm_bf16_cost(*t, M, N, K, s, cus) + sum;
+            if (cost < best) {
+                best = cost;
+                tile = t;
+                splits = s;
+            }
+        }
+    if (tile == nullptr) {
+        gemm_tile_launch<BLayout::nk, false, Epi, kStore>(rows.tile, A, W, bias, C, M, N, K, epi, stream);
         return false;
     }
-    // One workgroup per CU for the tall tiles, two for the small ones: split toward that many.
-    auto run = [&](auto shape, int target) {
+    auto run = [&](auto shape) {
         using S = decltype(shape);
-        const int tiles = static_cast<int>(blocks_for64(M, S::BM) * blocks_for64(N, S::BN));
-        int splits = 1;
-        if constexpr (!kSwiglu) {
-            splits = splitk_factor(tiles, static_cast<int>(blocks_for64(K, 64)), target);
-            if (N % 4 != 0 || !ws || int64_t(splits) * M * N > ws_floats || !aligned16(C) ||
-                (bias && !aligned16(bias)))
-                splits = 1;
-        }
+        const int64_t tiles = blocks_for64(M, S::BM) * blocks_for64(N, S::BN);
+        require(tiles <= INT32_MAX, "gemm_bf16: grid too large");
+        const dim3 grid(static_cast<unsigned>(tiles), static_cast<unsigned>(splits));
         if (splits == 1)
-            launch_async(stream, gemm_bf16_mfma_kernel<uint16_t, true, Epi, kStore, S>, dim3(tiles, 1), S::kThreads,
-                         A, W, bias, C, M, N, K, epi);
-        else
-            launch_async(stream, gemm_bf16_mfma_kernel<uint16_t, true, IdentityEpilogue, GemmStore::partial, S>,
-                         dim3(tiles, splits), S::kThreads, A, W, static_cast<const float *>(nullptr), ws, M, N, K,
-                         IdentityEpilogue{});
-        return splits;
+            launch_async(stream, gemm_bf16_mfma_kernel<Epi, kStore, S>, grid, S::kThreads, A, W, bias, C, M, N, K, epi);
+        else if constexpr (!kSwiglu)
+            launch_async(stream, gemm_bf16_mfma_kernel<IdentityEpilogue, GemmStore::partial, S>, grid, S::kThreads, A,
+                         W, static_cast<const float *>(nullptr), ws, M, N, K, IdentityEpilogue{});
     };
-    const int splits = M >= 256 ? run(BfTall{}, 256) : run(BfSmall{}, 512);
+    if (tile == &kGemmCostTall)
+        run(BfTall{});
+    else if (tile == &kGemmCostMid)
+        run(BfMid{});
+    else
+        run(BfBig{});
     if (splits == 1)
         return false;
-    if constexpr (!kSwiglu) {
-        if constexpr (std::is_same_v<Reduce, std::nullptr_t>)
-            launch_async(stream, splitk_reduce_kernel<Epi, kStore>, stream_grid(int64_t(M) * N / 4), 256, ws, splits,
-                         bias, C, M, N, epi);
-        else
-            reduce(ws, splits);
-    }
-    return true;
+    if constexpr (kHook)
+        reduce(ws, splits);
+    else if constexpr (!kSwiglu)
+        launch_async(stream, splitk_reduce_kernel<Epi, kStore>, stream_grid(int64_t(M) * N / 4), 256, ws, splits, bias,
+                     C, M, N, epi);
+    return kHook;
 }
 
 } // namespace opworks::detail

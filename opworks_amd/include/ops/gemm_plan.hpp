@@ -33,6 +33,7 @@ enum class GemmTile {
     staged16x16, // gemm_rows_kernel through LDS, rows on the 16-byte grid
     staged32x32,
     staged64x32,
+    staged64x64, // one bf16 part per operand
     direct16x16, // gemm_rows_kernel straight from memory, any alignment
     direct32x32,
     fp32_mfma, // gemm_f32_mfma_kernel
@@ -68,13 +69,29 @@ inline constexpr GemmTileCost kGemmCostWbf16[] = {
     {GemmTile::staged32x32, 32, 32, 1.6f, 2.2f, 0.18f},   {GemmTile::staged64x32, 64, 32, 1.35f, 3.6f, 0.305f},
     {GemmTile::direct16x16, 16, 16, 2.5f, 0.f, 0.091f},   {GemmTile::direct32x32, 32, 32, 4.5f, 0.f, 0.19f},
 };
+// fp32 X rounded to bf16, bf16 W. (64 x 128 tiles fitted by eye: few products ran fastest on them.)
+inline constexpr GemmTileCost kGemmCostRound[] = {
+    {GemmTile::parts128x256, 128, 256, 5.f, 0.f, 0.9f},   {GemmTile::parts64x128, 64, 128, 3.f, 3.f, 0.30f},
+    {GemmTile::parts64x64, 64, 64, 6.4f, 0.f, 0.243f},    {GemmTile::staged16x16, 16, 16, 1.25f, 1.f, 0.035f},
+    {GemmTile::staged32x32, 32, 32, 0.93f, 1.4f, 0.074f}, {GemmTile::staged64x32, 64, 32, 0.44f, 2.5f, 0.107f},
+    {GemmTile::staged64x64, 64, 64, 0.f, 4.35f, 0.126f},  {GemmTile::direct16x16, 16, 16, 1.94f, 0.f, 0.09f},
+    {GemmTile::direct32x32, 32, 32, 1.7f, 0.f, 0.18f},
+};
+// bf16 X and W; the parts tiles for operands off the 16-byte grid
+inline constexpr GemmTileCost kGemmCostBf16[] = {
+    {GemmTile::parts128x256, 128, 256, 5.4f, 0.f, 0.73f}, {GemmTile::parts64x64, 64, 64, 6.2f, 0.f, 0.204f},
+    {GemmTile::staged16x16, 16, 16, 1.9f, 0.45f, 0.023f}, {GemmTile::staged32x32, 32, 32, 0.87f, 1.35f, 0.053f},
+    {GemmTile::staged64x32, 64, 32, 0.36f, 2.3f, 0.069f}, {GemmTile::staged64x64, 64, 64, 0.f, 4.1f, 0.095f},
+    {GemmTile::direct16x16, 16, 16, 1.9f, 0.f, 0.07f},    {GemmTile::direct32x32, 32, 32, 1.5f, 0.f, 0.142f},
+};
 
 inline bool gemm_tile_is_parts(GemmTile t) {
     return t == GemmTile::parts128x256 || t == GemmTile::parts128x128 || t == GemmTile::parts64x128 ||
            t == GemmTile::parts64x64;
 }
 inline bool gemm_tile_is_staged(GemmTile t) {
-    return t == GemmTile::staged16x16 || t == GemmTile::staged32x32 || t == GemmTile::staged64x32;
+    return t == GemmTile::staged16x16 || t == GemmTile::staged32x32 || t == GemmTile::staged64x32 ||
+           t == GemmTile::staged64x64;
 }
 
 // The cheapest tile of `table`: the split-operand ones only with `parts`, the staged ones only with
@@ -122,11 +139,18 @@ void gemm_tile_launch(GemmTile tile, const TA *A, const TB *B, const float *bias
         if constexpr (std::is_same_v<TB, float>)
             parts(GemmParts128x128{});
         break;
-    case GemmTile::parts64x128: parts(GemmParts64x128{}); break;
+    case GemmTile::parts64x128:
+        if constexpr (std::is_same_v<TA, float>)
+            parts(GemmParts64x128{});
+        break;
     case GemmTile::parts64x64: parts(GemmParts64x64{}); break;
     case GemmTile::staged16x16: rows(GemmRows16x16{}, std::true_type{}); break;
     case GemmTile::staged32x32: rows(GemmRows32x32{}, std::true_type{}); break;
     case GemmTile::staged64x32: rows(GemmRows64x32{}, std::true_type{}); break;
+    case GemmTile::staged64x64:
+        if constexpr (std::is_same_v<TB, uint16_t> && (kRound || std::is_same_v<TA, uint16_t>))
+            rows(RowsShape<4, 4, 4, kRound ? 1 : 2>{}, std::true_type{});
+        break;
     case GemmTile::direct16x16: rows(GemmRows16x16{}, std::false_type{}); break;
     case GemmTile::direct32x32: rows(GemmRows32x32{}, std::false_type{}); break;
     case GemmTile::fp32_mfma: throw std::invalid_argument("gemm: the fp32-MFMA tiles have their own launcher");

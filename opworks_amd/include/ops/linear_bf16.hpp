@@ -33,8 +33,7 @@ inline void linear_bf16_validate(const TA *X, const uint16_t *W, float *Y, int r
     require(in_features > 0, "linear_mma_bf16 requires a positive reduction dim");
 }
 
-// Up to 64 rows: gemm_rows_kernel. Above, fp32 X: the register-staged GEMM (rounded as staged); bf16 X:
-// the direct-load GEMM on tiles sized to the row count (no workspace, so no split-K).
+// bf16 X on the 16-byte grid also has the direct-load tiles (no workspace, so no split-K).
 template <typename TA, typename Epi>
 inline void linear_bf16_launch(const TA *X, const uint16_t *W, const float *bias, float *Y, int rows, int in_features,
                                int out_features, Epi epi, hipStream_t stream) {
@@ -42,7 +41,7 @@ inline void linear_bf16_launch(const TA *X, const uint16_t *W, const float *bias
         gemm_bf16_launch_direct<Epi, GemmStore::store>(X, W, bias, Y, rows, out_features, in_features, epi, nullptr, 0,
                                                        stream);
     else
-        gemm_bf16_launch(X, W, bias, Y, rows, out_features, in_features, epi, stream);
+        gemm_bf16_launch<TA, Epi, GemmStore::store>(X, W, bias, Y, rows, out_features, in_features, epi, stream);
 }
 
 template <typename TA>

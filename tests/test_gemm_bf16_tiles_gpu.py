@@ -1,0 +1,50 @@
+"""The bf16 GEMM on each tile its cost model can pick, at sizes whose edges are partial (rows, columns, K
+tiles), for fp32 inputs (rounded) and bf16 inputs, and operands off the 16-byte grid.
+
+Tolerance: the rounded inputs' products are exact in fp32, and a sum of K terms in fp32 in any order is
+within (K + 1) 2^-23 of sum |a b| (the matrix core may truncate)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+# (M, out, inner)
+SIZES = [
+    (70, 304, 2288), (200, 2296, 552), (300, 4100, 520), (700, 2050, 1096),      # 16 x 16 ... 64 x 64
+    (129, 16384, 200), (513, 8200, 264), (1023, 4096, 264),                      # 128 x 256
+    (700, 16300, 264), (577, 16384, 72),                                         # 192 x 256
+    (4090, 4100, 72), (2050, 8190, 136),                                         # 256 x 256
+    (66, 5, 8), (129, 1, 16), (65, 64, 64),
+]
+RAGGED = [(70, 305, 2289), (143, 2301, 559), (435, 1441, 1513), (1237, 5621, 583), (70, 67, 3), (66, 9, 7),
+          (300, 1000, 9)]
+
+
+def _bf16(a):
+    u = np.ascontiguousarray(a, np.float32).view(np.uint32)
+    b = ((u.astype(np.uint64) + 0x7FFF + ((u >> 16) & 1)) >> 16).astype(np.uint16)
+    return b, (b.astype(np.uint32) << 16).view(np.float32)
+
+
+@pytest.mark.parametrize("m,n,k,shift", [(*s, 0) for s in SIZES + RAGGED] + [(*s, 1) for s in SIZES[:6] + RAGGED[:3]])
+@pytest.mark.parametrize("x_bf16", [False, True])
+def test_bf16_tiles(ow, m, n, k, shift, x_bf16):
+    rng = np.random.default_rng(m * 31 + n * 7 + k)
+    a, w = rng.standard_normal((m, k), np.float32), rng.standard_normal((n, k), np.float32)
+    bias = rng.uniform(-1, 1, n).astype(np.float32)
+    (ab, av), (wb, wv) = _bf16(a), _bf16(w)
+
+    def up(x):
+        return ow.DeviceBuffer.from_host(np.concatenate([np.zeros(shift, x.dtype), x.reshape(-1)])).offset(shift)
+
+    da, dw, db = up(ab if x_bf16 else a), up(wb), up(bias)
+    out = up(np.concatenate([np.full(m * n, 7, np.float32), np.full(8, 3, np.float32)]))
+    ow.ops.linear_bf16(da, dw, db, out, m, k, n, "relu", x_bf16)
+    got = out.to_host()
+    assert np.array_equal(got[m * n:], np.full(8, 3, np.float32))
+    got = got[:m * n].reshape(m, n)
+    av, wv = av.astype(np.float64), wv.astype(np.float64)
+    want = np.maximum(av @ wv.T + bias, 0)
+    bound = (k + 3) * 2.0 ** -23 * (np.abs(av) @ np.abs(wv).T + np.abs(bias)) + 1e-37
+    worst = float(np.max(np.abs(got - want) / bound))
+    assert worst <= 1.0, worst
