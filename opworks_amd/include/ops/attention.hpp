@@ -96,8 +96,8 @@ template <typename Combine> __device__ __forceinline__ float column_combine(floa
 // kDT = head_dim / 16 (16-wide head-dim tiles); kWaves = q heads handled by
 // one workgroup (a GQA group, or an 8-head slice of a larger one); kTiles =
 // adjacent query tiles per workgroup, one wave per (tile, head): with 2 every
-// staged K/V tile feeds twice as many MFMA chains (used when the grid still
-// fills every CU's four workgroup slots).
+// staged K/V tile feeds twice as many MFMA chains (used when the
+// one-tile grid overfills the CUs' workgroup slots).
 template <int kDT, int kWaves, int kTiles, bool kX6 = false> struct PrefillShape {
     static constexpr int kD = 16 * kDT;                        // head_dim
     static constexpr int kLd = kD + 4;                         // LDS row stride of K and V (floats)
@@ -724,12 +724,15 @@ inline void attention_prefill_launch(const float *q, const float *k, const float
                      cap, scale * kLog2e, pass_width, PrefillSplit{nullptr, nullptr, 0, 0}, ol);
 }
 
-// Two query tiles per workgroup when the one-tile grid would fill every CU's four
-// workgroup slots (measured on near-uniform work: 76 -> 79.5% of the MFMA peak); one
-// otherwise, so short prompts still spread over all CUs.
+// Two query tiles per workgroup when the one-tile grid overfills the CUs' workgroup slots, one otherwise,
+// so short prompts spread over all CUs. At head_dim 64 the LDS holds three one-tile workgroups per CU, and
+// two tiles, which share each staged and split K/V tile, win from 3.5 per CU, with or without cached keys
+// (32 q / 8 kv heads, one against two tiles: 1800 queries 94 -> 91 us, 2000 120 -> 106, 2000 behind 2000 cached keys
+// 336 -> 269; 16 heads without groups, 1000: 78 -> 51; but 1600 queries, 3.1 per CU, 75 -> 80). At head_dim 32
+// twice as many fit, and the line stays at four per CU (1600 queries 45 -> 52 us).
 template <int kDT, int kWaves> inline bool prefill_two_tiles(int T, int kv_rep, int kvh) {
     const int64_t wgs = blocks_for64(T, kAttnQTile) * kvh * ((kv_rep + kWaves - 1) / kWaves);
-    return wgs >= 4 * int64_t(cu_count());
+    return 2 * wgs >= (kDT == 4 ? 7 : 8) * int64_t(cu_count());
 }
 
 template <int kDT, int kWaves>
